@@ -387,3 +387,46 @@ def test_trajectories_match_oracle_loop(gpu, batch):
         same &= np.all(got[k] == want[k], axis=(1, 2))
     _log(f"  {int(same.sum())} of {reps} repetitions identical")
     assert same.mean() >= 0.999
+
+
+@pytest.mark.parametrize("m,shift", [(5, 0), (6, 1), (8, 0), (9, 1), (13, 0), (17, 0)])
+def test_draw_rows_at_ties_and_binade_edges(gpu, m, shift):
+    """cqs_draw_rows where adding elements out of order would round differently: elements half way
+    between two float64 values of the running sum, elements far below its last bit, sums that double
+    at every step, leading zeros, and uniforms on NumPy's own cdf values and beside them."""
+    _log(f"draw rows at ties m={m}")
+    import torch
+
+    from cirq_amd import engine
+
+    N = 2**m
+    rng = np.random.RandomState(m)
+    ties = np.zeros(N, dtype=np.float32)
+    ties[0] = ties[-1] = 0.5  # float32 sum 1: the elements stay as they are
+    ties[1:-1] = np.float32(2.0**-54) * rng.randint(0, 4, N - 2)
+    doubling = np.zeros(N, dtype=np.float32)
+    k = min(N, 60)
+    doubling[N - k:] = 2.0 ** np.arange(-k, 0)
+    doubling[N - 1] += np.float32(2.0**-k)
+    spread = (2.0 ** rng.uniform(-80, -m, N)).astype(np.float32)
+    single = np.zeros(N, dtype=np.float32)
+    single[N // 2] = 1
+    rows, us = [], []
+    for row in (ties, doubling, spread, single, rng.exponential(size=N).astype(np.float32)):
+        p = row / row.sum()
+        cdf = p.astype(np.float64).cumsum()
+        cdf /= cdf[-1]
+        for i in rng.randint(0, N, 6):
+            for u in (cdf[i], np.nextafter(cdf[i], 0), np.nextafter(cdf[i], 1)):
+                rows.append(row)
+                us.append(min(u, np.nextafter(1.0, 0)))
+    q, u = np.stack(rows), np.array(us)
+    buf = torch.empty(q.size + shift, dtype=torch.float32, device="cuda")
+    buf[shift:] = torch.from_numpy(q.reshape(-1)).cuda()
+    idx, p = engine.draw_rows(buf[shift:].view(q.shape), u, engine.Workspace(torch.device("cuda")))
+    for r in range(len(q)):
+        pr = q[r] / q[r].sum()
+        cdf = pr.astype(np.float64).cumsum()
+        cdf /= cdf[-1]
+        want = int(cdf.searchsorted(u[r], side="right"))  # RandomState.choice for the uniform u[r]
+        assert idx[r] == want and p[r] == pr[want], (r, idx[r], want)
