@@ -146,6 +146,15 @@ __global__ __launch_bounds__(256) void k_select_run(float2* __restrict__ amps, u
   }
   __syncthreads();
   const int copy = blockIdx.y;
+  // A copy that every op of the run leaves alone (selection out of range: the host marks a drawn
+  // identity so) is neither read nor written.  With 0.1% noise 99.6% of the copies of a run of four
+  // are: 512 copies of 16 qubits take 21 us a run against 135 us.
+  bool any = false;
+  for (int i = threadIdx.x & 15; i < R.nops; i += 16) {
+    const int sel = table[(size_t)srow[i] * n_states + copy];
+    any = any || (sel >= 0 && sel < snm[i]);
+  }
+  if (!__syncthreads_or(any)) return;
   float2* s = amps + (uint64_t)copy * per;
   const int D = 1 << R.u;
   const int t = threadIdx.x;

@@ -100,6 +100,7 @@ class TrajectoryBatch:
         self.n_draws = sum(1 for kind, _ in actions if kind == "op")
         self._channels: dict = {}  # stochastic op index -> its matrices on the device
         self._mix_mats: dict = {}  # stochastic op index -> its matrices (host complex64, flat)
+        self._identity: dict = {}  # stochastic op index -> which of its matrices are the identity
         self._plan = None  # the actions as steps, with runs of mixtures merged (built on first use)
 
     @staticmethod
@@ -177,6 +178,7 @@ class TrajectoryBatch:
             hit = (targets, m_dev, n_mats, probs)
             self._channels[j] = hit
             self._mix_mats[j] = mats.astype(np.complex64).reshape(-1)
+            self._identity[j] = np.all(mats.astype(np.complex64) == np.eye(mats.shape[-1]), axis=(1, 2))
         return hit
 
     def _steps(self):
@@ -245,7 +247,9 @@ class TrajectoryBatch:
         table = np.full((max(D, 1), R), -1, dtype=np.int32)
         for j, (targets, _, n_mats, probs) in self._channels.items():
             if probs is not None:
-                table[j] = choice_rows(np.broadcast_to(probs, (R, len(probs))), u[:, j])
+                drawn = choice_rows(np.broadcast_to(probs, (R, len(probs))), u[:, j])
+                # a drawn identity leaves the copy alone: -1, which the kernels do not touch
+                table[j] = np.where(self._identity[j][drawn], -1, drawn)
         table_dev = engine._dev_array(table, self.device)
         ones = torch.ones(R, dtype=torch.float32, device=self.device)
         u_dev = engine._dev_array(np.ascontiguousarray(u.T), self.device) if D else None  # row j: op j
@@ -267,9 +271,12 @@ class TrajectoryBatch:
             else:
                 ops = []
                 for j in step[1]:
+                    if (table[j] < 0).all():
+                        continue  # every copy drew the identity
                     targets, _, n_mats, _ = self._channels[j]
                     ops.append((len(targets), targets, self._run_offsets[j], n_mats, j))
-                engine.select_run_batch(states, self.n_bits, R, ops, self._run_mats, table_dev)
+                if ops:
+                    engine.select_run_batch(states, self.n_bits, R, ops, self._run_mats, table_dev)
         return recs
 
     def _measure(self, states, R: int, op, u: np.ndarray):
