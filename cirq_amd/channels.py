@@ -86,8 +86,8 @@ class AsymmetricDepolarizingChannel(Channel):
     def _mixture_(self):
         out = []
         for pauli, p in self._error_probabilities.items():
-            m = np.identity(1, dtype=np.complex128)
-            for c in pauli:
+            m = np.array(_PMAT[pauli[0]], dtype=np.complex128) if pauli else np.identity(1, dtype=np.complex128)
+            for c in pauli[1:]:
                 m = np.kron(m, _PMAT[c])
             out.append((p, m))
         return tuple(out)

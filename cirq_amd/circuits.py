@@ -486,12 +486,9 @@ def _needs_decompose(op) -> bool:
     (cirq-core/cirq/protocols/apply_unitary_protocol.py:375-389)."""
     if isinstance(op, CircuitOperation):
         return True
-    if _is_measurement(op):
-        return False
     g = getattr(op, "gate", None)
     obj = g if g is not None else op
-    dec = getattr(obj, "_decompose_", None)
-    if dec is None:
+    if getattr(obj, "_decompose_", None) is None or _is_measurement(op):
         return False
     if type(obj).__name__ in ("PauliString", "SingleQubitPauliStringGateOperation"):
         return False

@@ -452,12 +452,19 @@ class Sampler:
         return self._pbuf
 
     def bits(self, idx: torch.Tensor, m: int) -> np.ndarray:
-        reps = int(idx.shape[0])
-        out = torch.empty(max(reps * m, 1), dtype=torch.uint8, device=self.device)
-        check(lib().cqs_indices_to_bits(ptr(idx), reps, m, ptr(out), stream_handle()), "cqs_indices_to_bits")
+        return self.columns([(idx, range(m))], int(idx.shape[0]), m)
+
+    def columns(self, parts, reps: int, width: int) -> np.ndarray:
+        """uint8[reps, width] from parts (indices, columns): the big-endian digits of each part's
+        indices in its columns.  The parts cover every column."""
+        out = torch.empty(max(reps * width, 1), dtype=torch.uint8, device=self.device)
+        for idx, cols in parts:
+            c = np.array(list(cols), dtype=np.int32)
+            check(lib().cqs_indices_to_columns(ptr(idx), reps, len(c), c.ctypes.data, width, ptr(out), stream_handle()),
+                  "cqs_indices_to_columns")
         # one DMA copy into page-locked memory (torch's host allocator hands the block out again
         # once the returned array is dropped) instead of a staged copy into fresh pageable memory
         host = torch.empty(out.shape, dtype=torch.uint8, pin_memory=True)
         host.copy_(out, non_blocking=True)
         torch.cuda.current_stream().synchronize()
-        return host[: reps * m].numpy().reshape(reps, m)
+        return host[: reps * width].numpy().reshape(reps, width)

@@ -36,12 +36,23 @@ class Qid:
         return self._cmp_tuple() < other._cmp_tuple()
 
     def __eq__(self, other):
+        if self is other:
+            return True
         if not isinstance(other, Qid):
             return NotImplemented
         return self._cmp_tuple() == other._cmp_tuple()
 
     def __hash__(self):
-        return hash(self._cmp_tuple())
+        try:
+            return self._hash
+        except AttributeError:  # a qubit's key never changes; circuits look it up once per operation
+            self._hash = hash(self._cmp_tuple())
+            return self._hash
+
+    def __getstate__(self):
+        state = self.__dict__.copy()
+        state.pop("_hash", None)  # string hashes differ between processes
+        return state
 
 
 class LineQubit(Qid):

@@ -27,7 +27,7 @@ from . import engine
 from .channels import NoiseModel
 from .circuits import Circuit, Moment, expand_for_simulation
 from .gates import is_parameterized
-from .paulis import PauliSum, pauli_masks
+from .paulis import PauliString, PauliSum, pauli_masks
 from .qubits import QubitOrder
 from .study import ParamResolver, ResultDict, to_resolvers
 from .tape import (
@@ -410,11 +410,11 @@ class _SimulatorBase:
     # ---------------------------------------------------------------- sampling
     def _sample_factors(self, st, comp: _Compiled, factors, measured: list, reps: int) -> np.ndarray:
         """Samples `measured` qubits factor by factor with the simulator's prng; columns in measured order."""
-        mset = set(measured)
-        columns, order = [], []
+        column = {q: i for i, q in enumerate(measured)}
+        parts = []
         idx = {q: i for i, q in enumerate(comp.qubits)}
         for fq in factors:
-            qs = [q for q in fq if q in mset]
+            qs = [q for q in fq if q in column]
             if not qs:
                 continue
             u = self._prng.random_sample(reps)
@@ -426,25 +426,24 @@ class _SimulatorBase:
             else:
                 probs = self._sampler.marginal(st, comp.n, self._dm, axes)
                 ind = self._sampler.draw(None, len(axes), False, u, probs=probs)
-            columns.append(self._sampler.bits(ind, len(axes)))
-            order += qs
-        stacked = np.column_stack(columns) if columns else np.zeros((reps, 0), dtype=np.uint8)
-        pos = {q: i for i, q in enumerate(order)}
-        return stacked[:, [pos[q] for q in measured]]
+            parts.append((ind, [column[q] for q in qs]))
+        return self._sampler.columns(parts, reps, len(measured))
 
     def _records(self, bits: np.ndarray, measured: list, meas_ops) -> dict:
         qi = {q: i for i, q in enumerate(measured)}
         results: dict = {}
         for op in meas_ops:
             g = op.gate
-            out = np.zeros((bits.shape[0], len(op.qubits)), dtype=np.uint8)
-            inv = g.full_invert_mask() if hasattr(g, "full_invert_mask") else ()
-            for i, q in enumerate(op.qubits):
-                out[:, i] = bits[:, qi[q]]
-                if i < len(inv) and inv[i]:
-                    out[:, i] ^= 1
+            cols = [qi[q] for q in op.qubits]
+            first = cols[0] if cols else 0
+            adjacent = cols == list(range(first, first + len(cols)))
+            # a copy of its own: `bits` lies in page-locked memory that the next call reuses
+            out = bits[:, first : first + len(cols)].copy() if adjacent else np.ascontiguousarray(bits[:, cols])
+            inv = list(g.full_invert_mask())[: len(cols)] if hasattr(g, "full_invert_mask") else []
+            if any(inv):
+                out ^= np.array([bool(x) for x in inv] + [False] * (len(cols) - len(inv)), dtype=np.uint8)
             results.setdefault(g.key, []).append(out)
-        return {k: np.stack(v, axis=1) for k, v in results.items()}
+        return {k: v[0][:, None, :] if len(v) == 1 else np.stack(v, axis=1) for k, v in results.items()}
 
     # ---------------------------------------------------------------- SimulatesSamples
     def run(self, program, param_resolver=None, repetitions: int = 1) -> ResultDict:
@@ -798,8 +797,9 @@ class _SimulatorBase:
             else:
                 yield
 
-    def _needs_trajectory(self, circuit) -> bool:
-        if circuit.has_measurements() and not circuit.are_all_measurements_terminal():
+    def _needs_trajectory(self, circuit, measured: bool) -> bool:
+        """measured: whether the circuit has measurements."""
+        if measured and not circuit.are_all_measurements_terminal():
             return True
         return not self._dm and any(_has_channel(op) for op in circuit.all_operations())
 
@@ -807,7 +807,8 @@ class _SimulatorBase:
         resolvers = list(to_resolvers(params))
         circuit = self._noisy(program)
         qubits = QubitOrder.as_qubit_order(qubit_order).order_for(circuit.all_qubits())
-        if self._needs_trajectory(circuit):
+        measured = circuit.has_measurements()
+        if self._needs_trajectory(circuit, measured):
             actions = self._actions(circuit, qubits)
             for r in resolvers:
                 st = self._prepare_state(qubits, initial_state)
@@ -817,7 +818,7 @@ class _SimulatorBase:
                 meas = {k: (v[0] if len(v) == 1 else np.stack(v)) for k, v in records.items()}
                 yield self._trial_result(r, meas, st, _QubitsOnly(qubits))
             return
-        body, meas = _split_terminal_measurements(circuit)
+        body, meas = _split_terminal_measurements(circuit) if measured else (circuit, [])
         comp = self._compile(body, qubits)
         self._check_resolved(resolvers, comp)
         for r, st in zip(resolvers, self._run_program(comp, resolvers, initial_state)):
@@ -874,33 +875,31 @@ class _SimulatorBase:
             )
         if not isinstance(observables, list):
             observables = [observables]
-        pslist = [PauliSum.wrap(o) for o in observables]
         resolvers = list(to_resolvers(params))
         circuit = self._noisy(program)
         qubits = QubitOrder.as_qubit_order(qubit_order).order_for(circuit.all_qubits())
         qmap = {q: i for i, q in enumerate(qubits)}
         n = len(qubits)
         terms, owner = [], []
-        for oi, ps in enumerate(pslist):
-            for t in ps:
-                for q in t.qubits:
-                    if q not in qmap:
-                        raise KeyError(q)
-                terms.append(pauli_masks(t, qmap, n))
+        for oi, o in enumerate(observables):
+            # one string is its own only term; sums merge theirs
+            for t in (o,) if type(o) is PauliString else PauliSum.wrap(o):
+                terms.append(pauli_masks(t, qmap, n))  # KeyError for a qubit outside the circuit
                 owner.append(oi)
         owner = np.array(owner, dtype=np.int64)
 
         def values(st):
             vals = engine.expect_terms(st, n, self._dm, terms, self._ws).cpu().numpy()
-            sums = np.zeros(len(pslist), dtype=np.complex128)
+            sums = np.zeros(len(observables), dtype=np.complex128)
             np.add.at(sums, owner, vals)
             return [self._ev_value(v) for v in sums]
 
-        if self._needs_trajectory(circuit):
+        measured = circuit.has_measurements()
+        if self._needs_trajectory(circuit, measured):
             for res in self.simulate_sweep_iter(program, resolvers, qubits, initial_state):
                 yield values(res._state)
             return
-        body, meas = _split_terminal_measurements(circuit)
+        body, meas = _split_terminal_measurements(circuit) if measured else (circuit, [])
         comp = self._compile(body, qubits)
         self._check_resolved(resolvers, comp)
         for r, st in zip(resolvers, self._run_program(comp, resolvers, initial_state)):

@@ -92,9 +92,9 @@ def _is_pauli_string(op) -> bool:
 def _has_channel(op) -> bool:
     g = _gate_of(op)
     obj = g if g is not None else op
-    if getattr(obj, "_has_unitary_", lambda: False)() or is_parameterized(obj):
-        return False
-    return hasattr(obj, "_kraus_") or hasattr(obj, "_mixture_")
+    if not (hasattr(obj, "_kraus_") or hasattr(obj, "_mixture_")):
+        return False  # most ops: decided without evaluating their parameters
+    return not (getattr(obj, "_has_unitary_", lambda: False)() or is_parameterized(obj))
 
 
 def kraus_of(obj) -> list[np.ndarray]:

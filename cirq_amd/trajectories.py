@@ -101,6 +101,7 @@ class TrajectoryBatch:
         self._channels: dict = {}  # stochastic op index -> its matrices on the device
         self._mix_mats: dict = {}  # stochastic op index -> its matrices (host complex64, flat)
         self._identity: dict = {}  # stochastic op index -> which of its matrices are the identity
+        self._groups = None  # mixtures with equal probabilities (built on first use)
         self._plan = None  # the actions as steps, with runs of mixtures merged (built on first use)
 
     @staticmethod
@@ -237,6 +238,22 @@ class TrajectoryBatch:
         self._plan = steps
         return steps
 
+    def _mixture_groups(self):
+        """(normalised cdf, which matrices are the identity, op indices) of the mixtures, those with
+        equal probabilities and identities together: RandomState.choice searches the same float64
+        cdf for every copy and op of a group."""
+        if self._groups is None:
+            groups: dict = {}
+            for j, (_, _, _, probs) in self._channels.items():
+                if probs is not None:
+                    key = (probs.tobytes(), self._identity[j].tobytes())
+                    groups.setdefault(key, (probs, self._identity[j], []))[2].append(j)
+            self._groups = []
+            for probs, identity, js in groups.values():
+                cdf = np.cumsum(probs)
+                self._groups.append((cdf / cdf[-1], identity, np.array(js)))
+        return self._groups
+
     def _run_batch(self, state0: torch.Tensor, resolver, R: int, u: np.ndarray) -> list:
         copy_bits = R.bit_length() - 1
         states = state0.repeat(R)
@@ -245,11 +262,10 @@ class TrajectoryBatch:
         # known now and goes to the device in one copy (row j: stochastic op j)
         D = u.shape[1]
         table = np.full((max(D, 1), R), -1, dtype=np.int32)
-        for j, (targets, _, n_mats, probs) in self._channels.items():
-            if probs is not None:
-                drawn = choice_rows(np.broadcast_to(probs, (R, len(probs))), u[:, j])
-                # a drawn identity leaves the copy alone: -1, which the kernels do not touch
-                table[j] = np.where(self._identity[j][drawn], -1, drawn)
+        for cdf, identity, js in self._mixture_groups():
+            drawn = cdf.searchsorted(u[:, js].T, side="right")
+            # a drawn identity leaves the copy alone: -1, which the kernels do not touch
+            table[js] = np.where(identity[drawn], -1, drawn)
         table_dev = engine._dev_array(table, self.device)
         ones = torch.ones(R, dtype=torch.float32, device=self.device)
         u_dev = engine._dev_array(np.ascontiguousarray(u.T), self.device) if D else None  # row j: op j

@@ -486,6 +486,13 @@ int cqs_permuted_probs(const void* amps, int32_t n_qubits, int32_t is_dm, const 
  */
 int cqs_indices_to_bits(const int64_t* index, int64_t reps, int32_t m, uint8_t* out, void* stream);
 
+/*
+ * The same digits into chosen columns of rows of `width` bytes: out[r*width + columns[k]] = bit
+ * (m-1-k) of index[r] (columns: HOST, m entries in [0, width)); the other columns are left alone.
+ */
+int cqs_indices_to_columns(const int64_t* index, int64_t reps, int32_t m, const int32_t* columns, int32_t width,
+                           uint8_t* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -337,3 +337,24 @@ def test_passes_from_basis_state_match_init_then_passes(gpu, dm):
     want = torch.zeros(1 << nb, dtype=torch.complex64, device=dev)
     want[3] = 1
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("reps,widths", [(1, (1,)), (257, (5,)), (1000, (3, 1, 7)), (64, (62, 2))])
+def test_sample_digits_into_columns(gpu, reps, widths):
+    """Sampler.columns: each part's big-endian digits in its columns, in any order."""
+    import torch
+
+    from cirq_amd import engine
+
+    rng = np.random.RandomState(reps)
+    width = sum(widths)
+    order = rng.permutation(width)
+    parts, want, at = [], np.zeros((reps, width), dtype=np.uint8), 0
+    for m in widths:
+        idx = rng.randint(0, 2**m, reps, dtype=np.int64)
+        cols = [int(c) for c in order[at : at + m]]
+        for k, c in enumerate(cols):
+            want[:, c] = (idx >> (m - 1 - k)) & 1
+        parts.append((torch.from_numpy(idx).cuda(), cols))
+        at += m
+    assert np.array_equal(engine.Sampler(torch.device("cuda")).columns(parts, reps, width), want)
