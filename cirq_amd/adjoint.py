@@ -25,6 +25,7 @@ from .paulis import PauliSum, adjoint_scale, pauli_masks
 from .qubits import QubitOrder
 from .study import ParamResolver
 from .tape import (
+    Generator,
     LOp,
     Lowering,
     Pass,
@@ -52,9 +53,8 @@ def _dagger(kind: str, x):
 
 
 def _inverse(op: LOp, sel: int) -> LOp:
-    """U^dagger on the states `sel` selects.  The one-state inverses of a parameterised op and its
-    GRAD ops must share a pass: GRAD ops fold the controls into their matrix and need them local,
-    so the inverses ask for the same local bits.  (Split across passes, another op's gradient
+    """U^dagger on the states `sel` selects.  One-state inverses ask for their controls as local
+    bits too, so that the two of a pair share a pass.  (Split across passes, another op's gradient
     could run while only one of the two states had this inverse applied.)"""
     if op.kind == "scale" and abs(abs(complex(op.mat)) - 1) > 1e-9:
         raise ValueError("adjoint gradients need a unitary circuit (non-unit scale factor)")
@@ -66,25 +66,43 @@ def _inverse(op: LOp, sel: int) -> LOp:
     return LOp(op.kind, op.targets, _dagger(op.kind, op.mat), op.controls, ref, sel, need=need)
 
 
-def _grad_op(op: LOp, k: int, slot: int) -> LOp:
-    """d(op)/d(parameter k) as a GRAD op on the op's bits.
+def _constant_generator(gate):
+    """dM/dt M^dagger of a gate exp(i pi t K): i pi K, whatever t is; None for other gates."""
+    from .gates import EigenGate
 
-    The lowering's payload transforms are affine in the gate matrix (a controlled diagonal puts
-    constant ones outside the controlled block), so the derivative payload is
-    transform(dM) - transform(0).  Controls of a dense op are folded into its matrix the same way:
-    the blocks where the controls fail do not depend on the parameter."""
+    if not isinstance(gate, EigenGate) or type(gate)._dmatrix_batch is not EigenGate._dmatrix_batch:
+        return None
+    return sum(1j * np.pi * (h + gate._global_shift) * np.asarray(c, dtype=np.complex128)
+               for h, c in gate._eigen_components())
+
+
+def _grad_op(op: LOp, k: int, slot: int) -> LOp:
+    """The generator dU U^dagger of an op in its parameter k, as a GRAD op on the op's bits that runs
+    before the op is undone: 2 Re <phi_k| dU U^dagger |psi_k> is the derivative.
+
+    The lowering's payload transforms are affine in the gate matrix and keep products (a controlled
+    diagonal puts constant ones outside the controlled block), so the generator's payload is
+    transform(dM M^dagger) - transform(0).  Controls of a dense op are folded into its matrix the same
+    way: the blocks where the controls fail do not depend on the parameter."""
     ref = op.pref
     base = ref.transform
 
     def linear(b, base=base):
         return base(b) - base(np.zeros_like(b))
 
+    constant = _constant_generator(ref.gate)
+
+    def grad(kind, bits, transform):
+        if constant is not None:
+            return LOp(kind, bits, transform(constant[None])[0], (), None, 0, slot)
+        return LOp(kind, bits, None, (), ParamRef(ref.gate, transform, ref.exprs, ref.slot, Generator(k)), 0, slot)
+
     if op.kind == "diag":
-        return LOp("grad_diag", op.targets, None, (), ParamRef(ref.gate, linear, ref.exprs, ref.slot, k), 0, slot)
+        return grad("grad_diag", op.targets, linear)
     if op.kind != "dense":
         raise TypeError(f"cannot differentiate a {op.kind} op")
     if not op.controls:
-        return LOp("grad_dense", op.targets, None, (), ParamRef(ref.gate, linear, ref.exprs, ref.slot, k), 0, slot)
+        return grad("grad_dense", op.targets, linear)
     tb = list(op.targets)
     ctrls = tuple(op.controls)
     bits = tb + [b for b, _ in ctrls]
@@ -94,7 +112,7 @@ def _grad_op(op: LOp, k: int, slot: int) -> LOp:
         zero = embed(np.zeros_like(d[0]), tb, ctrls, bits)  # identity where the controls fail
         return np.stack([embed(x, tb, ctrls, bits) - zero for x in d])
 
-    return LOp("grad_dense", tuple(bits), None, (), ParamRef(ref.gate, controlled, ref.exprs, ref.slot, k), 0, slot)
+    return grad("grad_dense", tuple(bits), controlled)
 
 
 def default_tile_bits(n_bits: int) -> tuple[int, int]:
@@ -133,9 +151,9 @@ class AdjointProgram:
     from gradient slots to parameter expressions.  Needs no GPU.
 
     The reversed program walks the lowered ops backwards.  A fixed op U becomes U^dagger on both
-    states; a parameterised op becomes [U^dagger on psi][dU/dt_k for each symbolic parameter
-    t_k][U^dagger on phi].  Ops on disjoint bits commute, so the scheduler may move whole ops
-    across each other; each triple keeps its order because its members share their bits.
+    states; a parameterised op becomes [its generator for each symbolic parameter][U^dagger on both
+    states].  Ops on disjoint bits commute, so the scheduler may move whole ops across each other;
+    a gate's ops keep their order because they share their bits.
     """
 
     def __init__(self, circuit, observable, qubit_order=QubitOrder.DEFAULT, *, tile_bits: int | None = None,
@@ -175,13 +193,12 @@ class AdjointProgram:
             if op.fixed:
                 rev.append(_inverse(op, _lib.SEL_BOTH))
                 continue
-            rev.append(_inverse(op, _lib.SEL_PSI))
             for k, e in enumerate(op.pref.exprs):
                 if is_parameterized(e):
                     slot = len(self.grad_slots)
                     self.grad_slots.append((op.pref, k))
                     rev.append(_grad_op(op, k, slot))
-            rev.append(_inverse(op, _lib.SEL_PHI))
+            rev.append(_inverse(op, _lib.SEL_BOTH))
         rev = fuse_single_bit(rev)
         passes = schedule(rev, n, La, coalesce_bits)
         if mfma_blocks:

@@ -174,13 +174,12 @@ class DMAdjointProgram:
                 if op.fixed:
                     rev.append(_inverse(op, _lib.SEL_BOTH))
                     continue
-                rev.append(_inverse(op, _lib.SEL_PSI))
                 for k, e in enumerate(op.pref.exprs):
                     if is_parameterized(e):
                         slot = len(self.grad_slots)
                         self.grad_slots.append((op.pref, k))
                         rev.append(_grad_op(op, k, slot))
-                rev.append(_inverse(op, _lib.SEL_PHI))
+                rev.append(_inverse(op, _lib.SEL_BOTH))
             if chan is not None:
                 rev.append(_adjoint_of_nonunitary(chan))
             a = len(rev_passes)

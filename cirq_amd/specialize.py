@@ -234,6 +234,12 @@ def _adj_mixing(op, nt: int, per: int) -> bool:
     return kind in (_OP_DENSE, _lib.OP_GRAD_DENSE) and not _adj_register_dense(op, nt, per)
 
 
+def _in_diag_run(op) -> bool:
+    """adjoint.hpp in_diag_run: GRAD_DIAG, and DIAG or PAIRPHASE on both states."""
+    kind, sel = int(op["kind"]) & 0xFF, (int(op["kind"]) >> 8) & 3
+    return kind == _lib.OP_GRAD_DIAG or (kind in (_OP_DIAG, _OP_PAIR) and sel == 0)
+
+
 def _guard_cond(op) -> str:
     """The op's outer-control test as a C condition ('true' without outer controls)."""
     mask = int(op["co_mask_lo"]) | (int(op["co_mask_hi"]) << 32)
@@ -259,15 +265,28 @@ def adjoint_pass_source(index: int, ps, ops: np.ndarray) -> str:
         op = ops[first + j]
         kind, sel = int(op["kind"]) & 0xFF, (int(op["kind"]) >> 8) & 3
         ref = f"kA{index}_{j}"
+        if _in_diag_run(op):
+            run = ["  {\n    DiagRun<PER, NT> run;"]
+            while j < count and _in_diag_run(ops[first + j]):
+                op = ops[first + j]
+                kind, ref, cond = int(op["kind"]) & 0xFF, f"kA{index}_{j}", _guard_cond(op)
+                if kind == _lib.OP_GRAD_DIAG:
+                    run.append(f"    {{\n      double g = 0.0;\n      if (({cond}) && act) g = run.grad(va, vb, P, {ref}, base);\n"
+                               f"      write_wave_partial<NT>(g, partial, stride, tile, {int(op['slot'])});\n    }}")
+                else:
+                    guard = "" if cond == "true" else f"if ({cond}) "
+                    call = "ew_diag" if kind == _OP_DIAG else "ew_pairs"
+                    run.append(f"    {guard}{call}<PER, NT>(run.phases(), P, {ref}, base);")
+                j += 1
+            run.append("    run.finish(va, vb);\n  }")
+            body.append("\n".join(run))
+            continue
         if not _adj_mixing(op, nt, per):
             cond = _guard_cond(op)
-            if kind in (_lib.OP_GRAD_DIAG, _lib.OP_GRAD_DENSE):
-                if kind == _lib.OP_GRAD_DIAG:
-                    call = f"grad_reg_diag<PER, NT>(va, vb, P, {ref}, base)"
-                else:
-                    k = int(op["k"])
-                    r = [int(x) - tb for x in op["t"][:k]] + [0, 0]
-                    call = f"grad_reg_dense_k<PER, {k}, {r[0]}, {r[1]}, {r[2]}>(va, vb, scalar_ptr(P.mats) + {int(op['mat'])})"
+            if kind == _lib.OP_GRAD_DENSE:
+                k = int(op["k"])
+                r = [int(x) - tb for x in op["t"][:k]] + [0, 0]
+                call = f"grad_reg_dense_k<PER, {k}, {r[0]}, {r[1]}, {r[2]}>(va, vb, scalar_ptr(P.mats) + {int(op['mat'])})"
                 body.append(f"  {{\n    double g = 0.0;\n    if (({cond}) && act) g = {call};\n"
                             f"    write_wave_partial<NT>(g, partial, stride, tile, {int(op['slot'])});\n  }}")
                 j += 1

@@ -27,6 +27,23 @@ MAX_DIAG = 6
 OUTER = 64  # DIAG / PAIRPHASE bit encoding: tile-local index, or OUTER + global position
 
 
+@dataclasses.dataclass(frozen=True)
+class Generator:
+    """In ParamRef.deriv: evaluate dM/d(parameter k) M^dagger of the gate's matrix M."""
+
+    k: int
+
+
+def gate_matrices(gate, vals: tuple, deriv) -> np.ndarray:
+    """(B, d, d): the gate's matrices at the parameter values (deriv None), their derivatives in
+    parameter `deriv`, or the products of those with the inverse matrices (a Generator)."""
+    if deriv is None:
+        return np.asarray(gate._matrix_batch(vals))
+    if isinstance(deriv, Generator):
+        return gate._dmatrix_batch(vals, deriv.k) @ np.conj(np.swapaxes(gate._matrix_batch(vals), -1, -2))
+    return np.asarray(gate._dmatrix_batch(vals, deriv))
+
+
 @dataclasses.dataclass
 class ParamRef:
     """How to compute one lowered op's matrix from resolved parameter values.
@@ -39,7 +56,7 @@ class ParamRef:
     transform: Callable
     exprs: tuple
     slot: int = -1
-    deriv: int | None = None  # evaluate d(matrix)/d(parameter `deriv`) instead of the matrix
+    deriv: int | Generator | None = None  # evaluate a derivative or generator instead of the matrix
 
 
 @dataclasses.dataclass
@@ -894,8 +911,9 @@ class PackedProgram:
                     for m, b in enumerate(op.targets):
                         r["t"][m] = local[b]
                     d = 2**k
-                    r["mat"] = add_mat(np.zeros((d, d)))
-                    self.param_entries.append((int(r["mat"]), op.pref, d * d))
+                    r["mat"] = add_mat(np.zeros((d, d)) if op.mat is None else op.mat)
+                    if op.pref is not None:
+                        self.param_entries.append((int(r["mat"]), op.pref, d * d))
                     r["slot"] = op.slot
                 elif op.kind == "grad_diag":
                     k = len(op.targets)
@@ -903,8 +921,9 @@ class PackedProgram:
                     r["k"] = k
                     for m, b in enumerate(op.targets):
                         r["t"][m] = local[b] if b in local else OUTER + b
-                    r["mat"] = add_mat(np.zeros(2**k))
-                    self.param_entries.append((int(r["mat"]), op.pref, 2**k))
+                    r["mat"] = add_mat(np.zeros(2**k) if op.mat is None else op.mat)
+                    if op.pref is not None:
+                        self.param_entries.append((int(r["mat"]), op.pref, 2**k))
                     r["slot"] = op.slot
                 else:
                     raise ValueError(op.kind)
@@ -943,11 +962,13 @@ class PackedProgram:
             for op in ps.ops:
                 if op.kind == "pair":
                     run_pairs.append(op)
-                elif op.kind in ("dense", "block", "grad_dense", "grad_diag") or op.sel != 0:
+                elif op.kind in ("dense", "block", "grad_dense") or op.sel != 0:
                     flush()
                     ops.append(op)
                 else:
-                    ops.append(op)  # elementwise ops commute with the pending pair phases
+                    # elementwise ops commute with the pending pair phases, and a diagonal gradient
+                    # does not see phases applied to both states
+                    ops.append(op)
             flush()
             out.append(Pass(ps.L, ps.lpos, ops))
         return out
@@ -1438,9 +1459,7 @@ class ParamPlan:
     def _group_matrices(rep, exprs, symvals):
         """(G * B, d, d) matrices (or derivatives) of the group's gates, gate-major."""
         vals = tuple(e(symvals).reshape(-1) for e in exprs)
-        if rep.deriv is None:
-            return np.asarray(rep.gate._matrix_batch(vals))
-        return np.asarray(rep.gate._dmatrix_batch(vals, rep.deriv))
+        return gate_matrices(rep.gate, vals, rep.deriv)
 
     def __call__(self, symvals: np.ndarray) -> np.ndarray:
         B = symvals.shape[1]
@@ -1492,15 +1511,14 @@ def fill_param_mats_direct(prog: PackedProgram, ev: ParamEvaluator, symvals: np.
             for key in keys:
                 ref = refs[key]
                 vals = tuple(ev.values(e, symvals) for e in ref.exprs)
-                cache[key] = (ref.gate._matrix_batch(vals) if ref.deriv is None
-                              else ref.gate._dmatrix_batch(vals, ref.deriv))
+                cache[key] = gate_matrices(ref.gate, vals, ref.deriv)
             continue
         rep = refs[keys[0]]
         G = len(keys)
         vals = tuple(
             np.concatenate([ev.values(refs[key].exprs[p], symvals) for key in keys]) for p in range(len(rep.exprs))
         )
-        mb = rep.gate._matrix_batch(vals) if rep.deriv is None else rep.gate._dmatrix_batch(vals, rep.deriv)
+        mb = gate_matrices(rep.gate, vals, rep.deriv)
         mb = mb.reshape((G, B) + mb.shape[1:])
         for i, key in enumerate(keys):
             cache[key] = mb[i]
