@@ -18,6 +18,7 @@ LIB_PATH = Path(__file__).resolve().parent / "libcirq_amd.so"
 CQS_OK, CQS_ERR_ARG, CQS_ERR_HIP, CQS_ERR_OOM, CQS_ERR_UNSUPPORTED = 0, 1, 2, 3, 4
 OP_DENSE, OP_DIAG, OP_PAIRPHASE, OP_SCALE, OP_BLOCK = 1, 2, 3, 4, 5
 OP_GRAD_DENSE, OP_GRAD_DIAG, OP_PERMUTE = 6, 7, 8
+LANE_BITS = 6  # tile bits whose one-bit ops run across lanes (csrc/tile.hpp kLaneBits)
 SEL_BOTH, SEL_PSI, SEL_PHI = 0, 1, 2
 MAX_LOCAL = 16
 

@@ -149,8 +149,9 @@ __device__ __forceinline__ bool adj_register_dense(sop_t& op) {
   constexpr int TB = __builtin_ctz(NT);
   constexpr int NR = __builtin_ctz(PER);
   const int kind = op_kind(op);
-  if ((kind != CQS_OP_DENSE && kind != CQS_OP_GRAD_DENSE) || op.k < 1 || op.k > 3 || op.k > NR) return false;
-  if (op.t[0] < TB) return false;
+  if ((kind != CQS_OP_DENSE && kind != CQS_OP_GRAD_DENSE) || op.k < 1 || op.k > 3) return false;
+  if (op.t[0] < (op.k == 1 ? kLaneBits : 0)) return true;
+  if (op.k > NR || op.t[0] < TB) return false;
 #pragma unroll
   for (int m = 1; m < 3; ++m)
     if (m < op.k && op.t[m] <= op.t[m - 1]) return false;
@@ -199,12 +200,57 @@ __device__ __forceinline__ double grad_reg_dense_k(const float2 (&x)[PER], const
   return 2.0 * acc;
 }
 
+// 2 Re sum conj(f) G x over this thread's elements for a dense G on lane bit T: every lane weights its
+// own products and those with its partner's x by its row of G.
+template <int PER, int T>
+__device__ __forceinline__ double grad_lane1(const float2 (&x)[PER], const float2 (&f)[PER], smat_t* M) {
+  const float2 m00 = ldm(M, 0), m01 = ldm(M, 1), m10 = ldm(M, 2), m11 = ldm(M, 3);
+  const bool hi = (threadIdx.x >> T) & 1;
+  const float2 d = hi ? m11 : m00, o = hi ? m10 : m01;
+  double g = 0.0;
+  if (m00.x != 0.f || m11.x != 0.f) {
+    double s = 0.0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) s += (double)overlap<false>(f[e], x[e]);
+    g = fma((double)d.x, s, g);
+  }
+  if (m00.y != 0.f || m11.y != 0.f) {
+    double s = 0.0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) s += (double)overlap<true>(f[e], x[e]);
+    g = fma(-(double)d.y, s, g);
+  }
+  const bool re = m01.x != 0.f || m10.x != 0.f, im = m01.y != 0.f || m10.y != 0.f;
+  if (re || im) {
+    double sr = 0.0, si = 0.0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const float2 p = make_float2(lane_xor<T>(x[e].x), lane_xor<T>(x[e].y));
+      if (re) sr += (double)overlap<false>(f[e], p);
+      if (im) si += (double)overlap<true>(f[e], p);
+    }
+    g = fma((double)o.x, sr, g);
+    g = fma(-(double)o.y, si, g);
+  }
+  return 2.0 * g;
+}
+
 template <int PER, int NT, class Prog>
 __device__ __forceinline__ double grad_reg_dense(const float2 (&x)[PER], const float2 (&f)[PER], const Prog& P,
                                                  sop_t& op) {
   constexpr int TB = __builtin_ctz(NT);
   constexpr int NR = __builtin_ctz(PER);
   smat_t* M = scalar_ptr(P.mats) + op.mat;
+  if (op.k == 1 && op.t[0] < kLaneBits) {
+    switch (op.t[0]) {
+      case 0: return grad_lane1<PER, 0>(x, f, M);
+      case 1: return grad_lane1<PER, 1>(x, f, M);
+      case 2: return grad_lane1<PER, 2>(x, f, M);
+      case 3: return grad_lane1<PER, 3>(x, f, M);
+      case 4: return grad_lane1<PER, 4>(x, f, M);
+      default: return grad_lane1<PER, 5>(x, f, M);
+    }
+  }
   const int r0 = op.t[0] - TB, r1 = op.t[1] - TB, r2 = op.t[2] - TB;
   const int code = op.k == 1 ? r0 : (op.k == 2 ? 16 + r0 * 4 + r1 : 32 + r0 * 16 + r1 * 4 + r2);
 #define CQS_G1(A) \
@@ -362,7 +408,8 @@ __device__ __forceinline__ void adjoint_tile(float2* __restrict__ psi, float2* _
       }
       if (kind == CQS_OP_GRAD_DENSE) {
         double g = 0.0;
-        if (ok && act) g = grad_reg_dense<PER, NT>(va, vb, P, op);
+        if (ok) g = grad_reg_dense<PER, NT>(va, vb, P, op);  // exchanges lanes: every lane takes part
+        if (!act) g = 0.0;
         write_wave_partial<NT>(g, partial, stride, tile, op.slot);
         continue;
       }

@@ -48,10 +48,27 @@ def _shape(L: int) -> tuple[int, int]:
     return nt, per
 
 
+def _is_lane_op(op) -> bool:
+    """A one-bit op on a lane bit (tile.hpp kLaneBits), which runs across lanes in registers."""
+    return int(op["k"]) == 1 and int(op["t"][0]) < _lib.LANE_BITS
+
+
+def _reg_dense_call(op, state: str, mat: str, tb: int) -> str:
+    """A DENSE op that stays in registers (register or lane bits) on the elements `state`."""
+    k, cm, cv = int(op["k"]), int(op["cl_mask"]), int(op["cl_val"])
+    ctl = "true" if cm else "false"
+    if _is_lane_op(op):
+        return f"lane_reg_dense_k<PER, NT, {int(op['t'][0])}, {ctl}>({state}, {mat}, {cm}, {cv});"
+    r = [int(x) - tb for x in op["t"][:k]] + [0, 0]
+    return f"reg_dense_k<PER, NT, {k}, {r[0]}, {r[1]}, {r[2]}, {ctl}>({state}, {mat}, {cm}, {cv});"
+
+
 def _is_register_dense(op, nt: int, per: int) -> bool:
-    """tile.hpp is_register_dense: k <= 3 targets, all register bits, ascending."""
+    """tile.hpp is_register_dense: one lane bit, or k <= 3 targets, all register bits, ascending."""
     tb, nr = nt.bit_length() - 1, per.bit_length() - 1
     k = int(op["k"])
+    if (int(op["kind"]) & 0xFF) == _OP_DENSE and _is_lane_op(op):
+        return True
     if (int(op["kind"]) & 0xFF) != _OP_DENSE or k < 1 or k > 3 or k > nr:
         return False
     t = [int(x) for x in op["t"][:k]]
@@ -135,13 +152,9 @@ def pass_source(index: int, ps, ops: np.ndarray) -> str:
                 body.append(f"  __syncthreads();\n  regs_to_tile_permuted<PER, NT>(v, tile, L, scalar_ptr(P.aux) + {int(op['t'][0])}, act);\n"
                             "  __syncthreads();\n  tile_to_regs<PER, NT>(v, tile, act);")
             elif kind == _OP_DENSE:
-                k = int(op["k"])
-                r = [int(x) - tb for x in op["t"][:k]] + [0, 0]
                 var = _variant_expr(op)
-                mat = f"scalar_ptr(P.mats) + {int(op['mat'])}" + (f" + {var} * {1 << (2 * k)}" if var else "")
-                ctl = "true" if int(op["cl_mask"]) else "false"
-                body.append(f"  {guard}reg_dense_k<PER, NT, {k}, {r[0]}, {r[1]}, {r[2]}, {ctl}>(v, {mat}, "
-                            f"{int(op['cl_mask'])}, {int(op['cl_val'])});")
+                mat = f"scalar_ptr(P.mats) + {int(op['mat'])}" + (f" + {var} * {1 << (2 * int(op['k']))}" if var else "")
+                body.append(f"  {guard}" + _reg_dense_call(op, "v", mat, tb))
             elif kind == _OP_DIAG:
                 body.append(f"  {guard}ew_diag<PER, NT>(v, P, {ref}, base);")
             elif kind == _OP_PAIR:
@@ -218,9 +231,11 @@ extern "C" __global__ __launch_bounds__({nt}) __attribute__((amdgpu_waves_per_eu
 
 
 def _adj_register_dense(op, nt: int, per: int) -> bool:
-    """adjoint.hpp adj_register_dense: DENSE or GRAD_DENSE, k <= 3 register bits, ascending."""
+    """adjoint.hpp adj_register_dense: DENSE or GRAD_DENSE, one lane bit or k <= 3 register bits, ascending."""
     tb, nr = nt.bit_length() - 1, per.bit_length() - 1
     kind, k = int(op["kind"]) & 0xFF, int(op["k"])
+    if kind in (_OP_DENSE, _lib.OP_GRAD_DENSE) and _is_lane_op(op):
+        return True
     if kind not in (_OP_DENSE, _lib.OP_GRAD_DENSE) or k < 1 or k > 3 or k > nr:
         return False
     t = [int(x) for x in op["t"][:k]]
@@ -287,7 +302,9 @@ def adjoint_pass_source(index: int, ps, ops: np.ndarray) -> str:
                 k = int(op["k"])
                 r = [int(x) - tb for x in op["t"][:k]] + [0, 0]
                 call = f"grad_reg_dense_k<PER, {k}, {r[0]}, {r[1]}, {r[2]}>(va, vb, scalar_ptr(P.mats) + {int(op['mat'])})"
-                body.append(f"  {{\n    double g = 0.0;\n    if (({cond}) && act) g = {call};\n"
+                if _is_lane_op(op):
+                    call = f"grad_lane1<PER, {int(op['t'][0])}>(va, vb, scalar_ptr(P.mats) + {int(op['mat'])})"
+                body.append(f"  {{\n    double g = 0.0;\n    if ({cond}) g = {call};\n    if (!act) g = 0.0;\n"
                             f"    write_wave_partial<NT>(g, partial, stride, tile, {int(op['slot'])});\n  }}")
                 j += 1
                 continue
@@ -295,13 +312,9 @@ def adjoint_pass_source(index: int, ps, ops: np.ndarray) -> str:
             states = sel_states[sel]
             for st in states:
                 if kind == _OP_DENSE:
-                    k = int(op["k"])
-                    r = [int(x) - tb for x in op["t"][:k]] + [0, 0]
                     var = _variant_expr(op)
-                    mat = f"scalar_ptr(P.mats) + {int(op['mat'])}" + (f" + {var} * {1 << (2 * k)}" if var else "")
-                    ctl = "true" if int(op["cl_mask"]) else "false"
-                    body.append(f"  {guard}reg_dense_k<PER, NT, {k}, {r[0]}, {r[1]}, {r[2]}, {ctl}>({st}, {mat}, "
-                                f"{int(op['cl_mask'])}, {int(op['cl_val'])});")
+                    mat = f"scalar_ptr(P.mats) + {int(op['mat'])}" + (f" + {var} * {1 << (2 * int(op['k']))}" if var else "")
+                    body.append(f"  {guard}" + _reg_dense_call(op, st, mat, tb))
                 elif kind == _OP_DIAG:
                     body.append(f"  {guard}ew_diag<PER, NT>({st}, P, {ref}, base);")
                 elif kind == _OP_PAIR:

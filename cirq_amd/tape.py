@@ -981,8 +981,10 @@ def threads_for_tile(L: int) -> int:
 
 def order_tile_bits(p: Pass, coalesce: int) -> Pass:
     """Orders a pass's local bits: the coalescing bits first (thread lanes, contiguous in HBM),
-    then the rest by how many 1-2 bit dense ops use them, busiest last: the top
-    log2(2^L / threads) tile bits live in one thread's registers, where those ops skip LDS."""
+    then the rest by how many 1-2 bit dense ops use them: the busiest on top, where the
+    log2(2^L / threads) top tile bits live in one thread's registers and those ops skip LDS, then
+    the other lanes (one-bit ops skip LDS there too), the least used on the bits that number the
+    workgroup's waves."""
     L = p.L
     c = min(coalesce, L)
     low = [b for b in range(c) if b in p.lpos]
@@ -994,6 +996,9 @@ def order_tile_bits(p: Pass, coalesce: int) -> Pass:
                 if b in use:
                     use[b] += 1
     rest.sort(key=lambda b: (use[b], -b))
+    waves = max(0, min(threads_for_tile(L).bit_length() - 1, L) - _lib.LANE_BITS)
+    more_lanes = max(0, min(_lib.LANE_BITS, L) - len(low))
+    rest = rest[waves : waves + more_lanes] + rest[:waves] + rest[waves + more_lanes :]
     return Pass(L, tuple(sorted(low) + rest), p.ops)
 
 
@@ -1051,9 +1056,10 @@ def plan_registers(p: Pass, coalesce: int, costs: dict | None = None) -> Pass:
     dense ops whose targets are all register bits run there, other dense ops and MFMA blocks
     exchange the tile through LDS.  Ops are list-scheduled over their dependency graph (ops on
     disjoint bits commute, elementwise ops commute with each other): ready elementwise and
-    register ops run first; when only LDS ops are ready, the planner either re-lays the tile
-    (PERMUTE) so that a new set of register bits lets more ops run in registers, or runs the
-    ready op through LDS, whichever the cost table says is cheaper.  The coalescing bits stay the
+    register ops run first (one-bit ops on a lane bit, the six lowest tile bits, are such ops); when
+    only LDS ops are ready, the planner either re-lays the tile (PERMUTE) so that a new set of
+    register bits lets more ops run in registers, or runs the ready op through LDS, whichever the
+    cost table says is cheaper.  The coalescing bits stay the
     lowest tile bits throughout, so loads and stores remain contiguous."""
     costs = COSTS if costs is None else costs
     L = p.L
@@ -1074,8 +1080,14 @@ def plan_registers(p: Pass, coalesce: int, costs: dict | None = None) -> Pass:
             npred[j] += 1
     kmax_reg = min(3, NR)
 
+    lanes: set = set(low)  # bits now in lanes 0-5: their one-bit ops run across lanes
+
     def reg_ok(op, regs) -> bool:
-        return op.kind == "dense" and len(op.targets) <= kmax_reg and set(op.targets) <= regs
+        if op.kind != "dense":
+            return False
+        if len(op.targets) == 1 and op.targets[0] in lanes and op.targets[0] not in regs:
+            return True
+        return len(op.targets) <= kmax_reg and set(op.targets) <= regs
 
     def lds_cost(op) -> float:
         if op.kind == "dense":
@@ -1148,6 +1160,7 @@ def plan_registers(p: Pass, coalesce: int, costs: dict | None = None) -> Pass:
     S, _ = best_regs(npred, ready, done)
     start = low + [b for b in movable if b not in S] + sorted(S)
     layout = list(start)
+    lanes.update(start[: _lib.LANE_BITS])
     out: list[LOp] = []
 
     index_of = {id(op): j for j, op in enumerate(ops)}
@@ -1172,6 +1185,8 @@ def plan_registers(p: Pass, coalesce: int, costs: dict | None = None) -> Pass:
             S, gain = best_regs(npred, ready, done)
             if gain > costs["permute"]:
                 layout = layout_for(layout, S)
+                lanes.clear()
+                lanes.update(layout[: _lib.LANE_BITS])
                 out.append(LOp("permute", tuple(layout), None))
                 continue
             j = min(ready)
