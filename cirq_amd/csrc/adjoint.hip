@@ -1,6 +1,6 @@
 // Adjoint differentiation: one reverse sweep over psi (the forward state) and phi = H psi, FP64
 // per-tile partials reduced by cqs_grad_reduce.  The device code is in adjoint.hpp.
-#include "adjoint.hpp"
+#include "staged.hpp"
 
 namespace cqs {
 
@@ -15,9 +15,9 @@ __global__ __launch_bounds__(TileShape<L>::NT) __attribute__((amdgpu_waves_per_e
 
 typedef void (*AdjKernel)(float2*, float2*, TileProg, double*, int64_t);
 static const AdjKernel kAdjKernels[15] = {
-    k_adjoint_pass<0>, k_adjoint_pass<1>, k_adjoint_pass<2>,  k_adjoint_pass<3>,  k_adjoint_pass<4>,
-    k_adjoint_pass<5>, k_adjoint_pass<6>, k_adjoint_pass<7>,  k_adjoint_pass<8>,  k_adjoint_pass<9>,
-    k_adjoint_pass<10>, k_adjoint_pass<11>, k_adjoint_pass<12>, k_adjoint_pass<13>, k_adjoint_pass<14>};
+    k_adjoint_pass<0>, k_adjoint_pass<1>, k_adjoint_pass<2>, k_adjoint_pass<3>,  k_adjoint_pass<4>,
+    k_adjoint_pass<5>, nullptr,           nullptr,           nullptr,            nullptr,
+    nullptr,           nullptr,           k_adjoint_pass<12>, k_adjoint_pass<13>, k_adjoint_pass<14>};  // 6-11: kAdjStaged
 
 // out[g] = sum_t partial[g * ntiles + t]  (fixed order)
 __global__ __launch_bounds__(64) void k_grad_reduce(const double* __restrict__ partial, int64_t ntiles,
@@ -58,11 +58,13 @@ static int adjoint_passes(void* psi, void* phi, int32_t n_bits, const cqs_pass* 
                 (long long)entries);
     const int mk = ps.max_k;
     const size_t stage = mk >= 3 ? (size_t(1) << (2 * mk)) : 0;
-    const size_t shmem = (2 * (size_t)tile_words(ps.L) + stage) * sizeof(float2);
+    const bool staged = kernels == nullptr && staged_adjoint_width(ps.L);
+    const size_t shmem =
+        (2 * (size_t)tile_words(ps.L) + stage) * sizeof(float2) + (staged ? kStagedBytes : 0);
+    const AdjKernel kernel = staged ? kAdjStaged[ps.L] : kAdjKernels[ps.L];
     CQS_REQUIRE(shmem <= 160 * 1024 - 1024, "adjoint pass needs %zu bytes of LDS", shmem);
     if (shmem > 64 * 1024)
-      CQS_HIP(hipFuncSetAttribute((const void*)kAdjKernels[ps.L], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)shmem));
+      CQS_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
     const int nt = ps.L <= 12 ? 256 : (1 << ps.L) / 16;
     if (kernels != nullptr) {
       CQS_REQUIRE(kernels[i] != nullptr, "no specialised kernel for reverse pass %d", i);
@@ -73,7 +75,7 @@ static int adjoint_passes(void* psi, void* phi, int32_t n_bits, const cqs_pass* 
       void* args[] = {&a, &b, &P, &grad_partial, &partial_stride};
       CQS_HIP(hipLaunchKernel(kernels[i], dim3((unsigned)tiles), dim3(nt), args, shmem, s));
     } else {
-      hipLaunchKernelGGL(kAdjKernels[ps.L], dim3((unsigned)tiles), dim3(nt), shmem, s, (float2*)psi, (float2*)phi,
+      hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(nt), shmem, s, (float2*)psi, (float2*)phi,
                          P, grad_partial, partial_stride);
     }
     CQS_HIP(hipGetLastError());

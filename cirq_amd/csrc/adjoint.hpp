@@ -34,8 +34,8 @@ __device__ __forceinline__ float overlap(float2 f, float2 x) {
 // 2 Re sum over pairs (m, n) of one bit of conj(f) M x, for a 2x2 M: the products that M's nonzero
 // parts need, summed over this thread's pairs, then weighted.  x(i, bit), f(i, bit): pair i's
 // amplitudes.
-template <class X, class F>
-__device__ __forceinline__ double grad_pairs(int pairs, X x, F f, smat_t* M) {
+template <class X, class F, class MPtr>
+__device__ __forceinline__ double grad_pairs(int pairs, X x, F f, MPtr M) {
   double g = 0.0;
 #pragma unroll
   for (int r = 0; r < 2; ++r)
@@ -60,9 +60,9 @@ __device__ __forceinline__ double grad_pairs(int pairs, X x, F f, smat_t* M) {
 
 // This thread's share (its groups) of 2 Re sum conj(phi) G psi over the LDS tiles for a dense G on
 // one tile bit.
-template <int NT, class Op>
-__device__ __forceinline__ double grad_dense1(const float2* psi, const float2* phi, int L, Op& op, smat_t* M) {
-  const int t = op.t[0], pt = pad(1 << t);
+template <int NT, class MPtr>
+__device__ __forceinline__ double grad_dense1(const float2* psi, const float2* phi, int L, int t, MPtr M) {
+  const int pt = pad(1 << t);
   const int pairs = ((1 << L) >> 1) / NT;
   double g = 0.0;
   if (pairs == 0) {  // fewer pairs than threads
@@ -95,7 +95,7 @@ __device__ __forceinline__ double grad_dense1(const float2* psi, const float2* p
 // (k <= 3) on tile bits op.t.
 template <int K, int NT, class Op>
 __device__ __forceinline__ double grad_dense(const float2* psi, const float2* phi, int L, Op& op, smat_t* M) {
-  if constexpr (K == 1) return grad_dense1<NT>(psi, phi, L, op, M);
+  if constexpr (K == 1) return grad_dense1<NT>(psi, phi, L, op.t[0], M);
   constexpr int D = 1 << K;
   int ts[K];
 #pragma unroll
@@ -168,8 +168,8 @@ __device__ __forceinline__ bool adj_mixing(sop_t& op) {
 // 2 Re sum conj(f) G x over this thread's groups of a register-bit dense G (targets R0 < R1 < R2,
 // matrix index bit m <-> target m): one bit through grad_pairs; more bits with G x in FP32 and the
 // products with conj(f) summed in FP64.
-template <int PER, int K, int R0, int R1, int R2>
-__device__ __forceinline__ double grad_reg_dense_k(const float2 (&x)[PER], const float2 (&f)[PER], smat_t* M) {
+template <int PER, int K, int R0, int R1, int R2, class MPtr>
+__device__ __forceinline__ double grad_reg_dense_k(const float2 (&x)[PER], const float2 (&f)[PER], MPtr M) {
   if constexpr (K == 1) {
     auto at = [](int i, int b) { return ((i >> R0) << (R0 + 1)) | (i & ((1 << R0) - 1)) | (b << R0); };
     return grad_pairs(PER / 2, [&](int i, int b) { return x[at(i, b)]; }, [&](int i, int b) { return f[at(i, b)]; }, M);
@@ -202,8 +202,8 @@ __device__ __forceinline__ double grad_reg_dense_k(const float2 (&x)[PER], const
 
 // 2 Re sum conj(f) G x over this thread's elements for a dense G on lane bit T: every lane weights its
 // own products and those with its partner's x by its row of G.
-template <int PER, int T>
-__device__ __forceinline__ double grad_lane1(const float2 (&x)[PER], const float2 (&f)[PER], smat_t* M) {
+template <int PER, int T, class MPtr>
+__device__ __forceinline__ double grad_lane1(const float2 (&x)[PER], const float2 (&f)[PER], MPtr M) {
   const float2 m00 = ldm(M, 0), m01 = ldm(M, 1), m10 = ldm(M, 2), m11 = ldm(M, 3);
   const bool hi = (threadIdx.x >> T) & 1;
   const float2 d = hi ? m11 : m00, o = hi ? m10 : m01;
@@ -272,11 +272,13 @@ __device__ __forceinline__ double grad_reg_dense(const float2 (&x)[PER], const f
 
 // A run of diagonal ops on both states (x: psi, f: phi): the products w_j = Im conj(f_j) x_j, formed
 // at the run's first GRAD_DIAG, serve all of them, and the run's phases are multiplied into the
-// states once, when it ends.
+// states once, when it ends.  The phases' product is kept in FP64: rounded to FP32 after every op, elements
+// with equal phases would all drift alike, and the run's rounding errors would add up instead of averaging
+// out (QAOA gradient off by 7e-6 instead of 2e-6).
 template <int PER, int NT>
 struct DiagRun {
   float w[PER];
-  float2 ph[PER];
+  double2 ph[PER];
   bool have_w = false, have_ph = false;
 
   // 2 Re sum conj(f_j) d(j) x_j for a diagonal d.  A generator's entries are imaginary: only w is
@@ -310,10 +312,10 @@ struct DiagRun {
     return 2.0 * acc;
   }
   // The run's phases, to be multiplied by a diagonal op's (ew_diag, ew_pairs).
-  __device__ __forceinline__ float2 (&phases())[PER] {
+  __device__ __forceinline__ double2 (&phases())[PER] {
     if (!have_ph) {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) ph[e] = make_float2(1.f, 0.f);
+      for (int e = 0; e < PER; ++e) ph[e] = make_double2(1.0, 0.0);
       have_ph = true;
     }
     return ph;
@@ -322,8 +324,9 @@ struct DiagRun {
     if (!have_ph) return;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      x[e] = cmul(x[e], ph[e]);
-      f[e] = cmul(f[e], ph[e]);
+      const float2 p = make_float2((float)ph[e].x, (float)ph[e].y);
+      x[e] = cmul(x[e], p);
+      f[e] = cmul(f[e], p);
     }
   }
 };
@@ -348,12 +351,88 @@ __device__ __forceinline__ void write_wave_partial(double g, double* __restrict_
 // per-slot partial entries).
 __host__ __device__ constexpr int adjoint_waves(int L) { return (L <= 12 ? 256 : (1 << L) / 16) / 64; }
 
+// One op of a register phase on this thread's elements of both states (a diagonal gradient alone:
+// adjoint_tile keeps runs together).
+template <int PER, int NT, class Prog>
+__device__ __forceinline__ void adjoint_register_op(float2 (&va)[PER], float2 (&vb)[PER], const Prog& P, sop_t& op,
+                                                    uint64_t base, bool act, double* __restrict__ partial,
+                                                    int64_t stride, int64_t tile) {
+  const int kind = op_kind(op), sel = op_sel(op);
+  const bool ok = outer_controls_ok(op, base);
+  if (kind == CQS_OP_GRAD_DIAG) {
+    DiagRun<PER, NT> run;
+    double g = 0.0;
+    if (ok && act) g = run.grad(va, vb, P, op, base);
+    write_wave_partial<NT>(g, partial, stride, tile, op.slot);
+    return;
+  }
+  if (kind == CQS_OP_GRAD_DENSE) {
+    double g = 0.0;
+    if (ok) g = grad_reg_dense<PER, NT>(va, vb, P, op);  // exchanges lanes: every lane takes part
+    if (!act) g = 0.0;
+    write_wave_partial<NT>(g, partial, stride, tile, op.slot);
+    return;
+  }
+  if (!ok) return;
+  if (kind == CQS_OP_DENSE) {
+    if (sel != kSelPhi) reg_dense<PER, NT>(va, P, op, base);
+    if (sel != kSelPsi) reg_dense<PER, NT>(vb, P, op, base);
+  } else if (kind == CQS_OP_DIAG) {
+    if (sel != kSelPhi) ew_diag<PER, NT>(va, P, op, base);
+    if (sel != kSelPsi) ew_diag<PER, NT>(vb, P, op, base);
+  } else if (kind == CQS_OP_PAIRPHASE) {
+    if (sel != kSelPhi) ew_pairs<PER, NT>(va, P, op, base);
+    if (sel != kSelPsi) ew_pairs<PER, NT>(vb, P, op, base);
+  } else if (kind == CQS_OP_SCALE) {
+    if (sel != kSelPhi) ew_scale<PER>(va, P, op);
+    if (sel != kSelPsi) ew_scale<PER>(vb, P, op);
+  }
+}
+
+// One op of an LDS phase on both LDS tiles.  The caller fences before.
+template <int NT, int L, class Prog>
+__device__ __forceinline__ void adjoint_mixing_op(float2* tA, float2* tB, float2* mstage, const Prog& P, sop_t& op,
+                                                  uint64_t base, double* __restrict__ partial, int64_t stride,
+                                                  int64_t tile) {
+  const int kind = op_kind(op), sel = op_sel(op);
+  const bool ok = outer_controls_ok(op, base);
+  if (kind == CQS_OP_GRAD_DENSE) {
+    double g = 0.0;
+    if (ok) {
+      smat_t* M = scalar_ptr(P.mats) + op.mat;
+      if (op.k == 1)
+        g = grad_dense<1, NT>(tA, tB, L, op, M);
+      else if (op.k == 2)
+        g = grad_dense<2, NT>(tA, tB, L, op, M);
+      else if (op.k == 3)
+        g = grad_dense<3, NT>(tA, tB, L, op, M);
+    }
+    write_wave_partial<NT>(g, partial, stride, tile, op.slot);
+    return;
+  }
+  if (!ok) return;
+  if (sel != kSelPhi) run_mixing_op<NT>(tA, mstage, P, op, base);
+  if (sel == kSelBoth) __syncthreads();  // the matrix stage is shared by both tiles
+  if (sel != kSelPsi) run_mixing_op<NT>(tB, mstage, P, op, base);
+}
+
+struct RunAdjoint {  // the interpreter below
+  template <int PER, int NT, int L, class Prog>
+  static __device__ __forceinline__ void run(float2 (&va)[PER], float2 (&vb)[PER], float2* tA, float2* tB,
+                                             float2* mstage, const Prog& P, uint64_t base, bool act,
+                                             double* __restrict__ partial, int64_t stride, int64_t tile);
+  template <int NT, class Prog>
+  static __device__ __forceinline__ void begin(const Prog& P, uint64_t, float2*) {
+    warm_program<NT>(P);
+  }
+};
+
 // One workgroup's share of a reverse-sweep pass.  psi and phi stay in registers (this thread's
 // elements, natural layout) through runs of elementwise ops, register-bit dense ops and GRAD ops on
 // register bits; ops that mix elements of different threads (other dense ops, MFMA blocks, GRAD
 // ops on thread bits) run on the two LDS tiles between barriers.  GRAD ops write one FP64 partial
 // per wave.  `stride` is the per-slot partial stride (tiles x waves).
-template <int L, class Prog>
+template <int L, class Run = RunAdjoint, class Prog>
 __device__ __forceinline__ void adjoint_tile(float2* __restrict__ psi, float2* __restrict__ phi, const Prog& P,
                                              const int32_t* lpos, uint64_t base, double* __restrict__ partial,
                                              int64_t stride, int64_t tile, float2* lds) {
@@ -362,7 +441,7 @@ __device__ __forceinline__ void adjoint_tile(float2* __restrict__ psi, float2* _
   float2* tB = lds + tile_words(L);
   float2* mstage = lds + 2 * tile_words(L);
   const bool act = L >= 8 || (int)threadIdx.x < (1 << L);
-  warm_program<NT>(P);
+  Run::template begin<NT>(P, base, mstage);
   float2 va[PER], vb[PER];
   {  // offsets are recomputed for the store, so they are not live across the program
     uint64_t off_lo, off_hi[PER];
@@ -378,13 +457,27 @@ __device__ __forceinline__ void adjoint_tile(float2* __restrict__ psi, float2* _
       for (int e = 0; e < PER; ++e) va[e] = vb[e] = make_float2(0.f, 0.f);
     }
   }
+  Run::template run<PER, NT, L>(va, vb, tA, tB, mstage, P, base, act, partial, stride, tile);
+  uint64_t off_lo, off_hi[PER];
+  tile_offsets<L>(lpos, off_lo, off_hi);
+  if (act) {
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      psi[base + off_lo + off_hi[e]] = va[e];
+      phi[base + off_lo + off_hi[e]] = vb[e];
+    }
+  }
+}
+
+template <int PER, int NT, int L, class Prog>
+__device__ __forceinline__ void RunAdjoint::run(float2 (&va)[PER], float2 (&vb)[PER], float2* tA, float2* tB,
+                                                float2* mstage, const Prog& P, uint64_t base, bool act,
+                                                double* __restrict__ partial, int64_t stride, int64_t tile) {
   int i = 0;
   for (;;) {
     // register phase
     for (; i < P.op_count && !adj_mixing<PER, NT>(scalar_ptr(P.ops)[i]); ++i) {
       sop_t& op = scalar_ptr(P.ops)[i];
-      const int kind = op_kind(op), sel = op_sel(op);
-      const bool ok = outer_controls_ok(op, base);
       if (in_diag_run(op)) {
         DiagRun<PER, NT> run;
         for (;; ++i) {
@@ -406,27 +499,7 @@ __device__ __forceinline__ void adjoint_tile(float2* __restrict__ psi, float2* _
         run.finish(va, vb);
         continue;
       }
-      if (kind == CQS_OP_GRAD_DENSE) {
-        double g = 0.0;
-        if (ok) g = grad_reg_dense<PER, NT>(va, vb, P, op);  // exchanges lanes: every lane takes part
-        if (!act) g = 0.0;
-        write_wave_partial<NT>(g, partial, stride, tile, op.slot);
-        continue;
-      }
-      if (!ok) continue;
-      if (kind == CQS_OP_DENSE) {
-        if (sel != kSelPhi) reg_dense<PER, NT>(va, P, op, base);
-        if (sel != kSelPsi) reg_dense<PER, NT>(vb, P, op, base);
-      } else if (kind == CQS_OP_DIAG) {
-        if (sel != kSelPhi) ew_diag<PER, NT>(va, P, op, base);
-        if (sel != kSelPsi) ew_diag<PER, NT>(vb, P, op, base);
-      } else if (kind == CQS_OP_PAIRPHASE) {
-        if (sel != kSelPhi) ew_pairs<PER, NT>(va, P, op, base);
-        if (sel != kSelPsi) ew_pairs<PER, NT>(vb, P, op, base);
-      } else if (kind == CQS_OP_SCALE) {
-        if (sel != kSelPhi) ew_scale<PER>(va, P, op);
-        if (sel != kSelPsi) ew_scale<PER>(vb, P, op);
-      }
+      adjoint_register_op<PER, NT>(va, vb, P, op, base, act, partial, stride, tile);
     }
     if (i >= P.op_count) break;
     // LDS phase: both tiles out of registers, then every consecutive op that mixes threads
@@ -435,39 +508,11 @@ __device__ __forceinline__ void adjoint_tile(float2* __restrict__ psi, float2* _
     for (; i < P.op_count && adj_mixing<PER, NT>(scalar_ptr(P.ops)[i]); ++i) {
       sop_t& op = scalar_ptr(P.ops)[i];
       __syncthreads();
-      const int kind = op_kind(op), sel = op_sel(op);
-      const bool ok = outer_controls_ok(op, base);
-      if (kind == CQS_OP_GRAD_DENSE) {
-        double g = 0.0;
-        if (ok) {
-          smat_t* M = scalar_ptr(P.mats) + op.mat;
-          if (op.k == 1)
-            g = grad_dense<1, NT>(tA, tB, L, op, M);
-          else if (op.k == 2)
-            g = grad_dense<2, NT>(tA, tB, L, op, M);
-          else if (op.k == 3)
-            g = grad_dense<3, NT>(tA, tB, L, op, M);
-        }
-        write_wave_partial<NT>(g, partial, stride, tile, op.slot);
-        continue;
-      }
-      if (!ok) continue;
-      if (sel != kSelPhi) run_mixing_op<NT>(tA, mstage, P, op, base);
-      if (sel == kSelBoth) __syncthreads();  // the matrix stage is shared by both tiles
-      if (sel != kSelPsi) run_mixing_op<NT>(tB, mstage, P, op, base);
+      adjoint_mixing_op<NT, L>(tA, tB, mstage, P, op, base, partial, stride, tile);
     }
     __syncthreads();
     tile_to_regs<PER, NT>(va, tA, act);
     tile_to_regs<PER, NT>(vb, tB, act);  // each thread reads back only its own slots: no barrier until the next mix
-  }
-  uint64_t off_lo, off_hi[PER];
-  tile_offsets<L>(lpos, off_lo, off_hi);
-  if (act) {
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      psi[base + off_lo + off_hi[e]] = va[e];
-      phi[base + off_lo + off_hi[e]] = vb[e];
-    }
   }
 }
 

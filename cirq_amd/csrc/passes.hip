@@ -6,7 +6,7 @@
 #include <unordered_map>
 #include <vector>
 
-#include "tile.hpp"
+#include "staged.hpp"
 
 namespace cqs {
 
@@ -437,6 +437,12 @@ static int run_passes(void* amps, int32_t n_bits, int64_t basis, const cqs_pass*
       void* args[] = {&psi, &P};
       CQS_HIP(hipLaunchKernel(kernels[i], dim3((unsigned)tiles), dim3(threads_for_L(ps.L)), args, shmem, s));
     } else {
+      if (staged_pass(P)) {  // at most 34 + 8 + 4 KB of LDS: within the default grant
+        hipLaunchKernelGGL(kPassStaged[ps.L], dim3((unsigned)tiles), dim3(threads_for_L(ps.L)),
+                           shmem + kStagedBytes, s, (float2*)amps, P);
+        CQS_HIP(hipGetLastError());
+        continue;
+      }
       if (int rc = ensure_pass_lds(ps.L, shmem)) return rc;
       hipLaunchKernelGGL(kPassKernels[ps.L], dim3((unsigned)tiles), dim3(threads_for_L(ps.L)), shmem, s,
                          (float2*)amps, P);

@@ -57,6 +57,8 @@ struct ProgView {
 constexpr int kPadShift = 5;
 __device__ __forceinline__ int pad(int j) { return j + (j >> kPadShift); }
 __host__ __device__ constexpr int tile_words(int L) { return (1 << L) + ((1 << L) >> kPadShift); }
+// float2 slots of the LDS stage for three-bit matrices.
+__host__ __device__ constexpr int mstage_words(int max_k) { return max_k >= 3 ? 1 << (2 * max_k) : 0; }
 // pad(threadIdx.x + e * NT) for NT a multiple of 2^kPadShift: one per-thread base plus a constant
 // per element (which the LDS instructions take as an immediate offset).
 template <int NT>
@@ -82,6 +84,11 @@ __device__ __forceinline__ float2 ldm(smat_t* p, int i) {
   return make_float2(f[2 * i], f[2 * i + 1]);
 }
 __device__ __forceinline__ float2 ldm(const float2* p, int i) { return p[i]; }
+// or held in registers
+struct Mat2 {
+  float2 m[4];
+};
+__device__ __forceinline__ float2 ldm(const Mat2& M, int i) { return M.m[i]; }
 
 // Bit encoding of DIAG / PAIRPHASE positions: values < kOuter are tile-local indices, values
 // >= kOuter are kOuter + a global position outside the tile.
@@ -459,8 +466,8 @@ struct DiagTable {
   __device__ __forceinline__ float2 at(int e) const { return small ? pick(index(e)) : Dg[index(e)]; }
 };
 
-template <int PER, int NT, class Prog, class Op>
-__device__ __forceinline__ void ew_diag(float2 (&v)[PER], const Prog& P, Op& op, uint64_t base) {
+template <int PER, int NT, class Prog, class Op, class C>
+__device__ __forceinline__ void ew_diag(C (&v)[PER], const Prog& P, Op& op, uint64_t base) {
   const DiagTable<PER, NT, Prog> D(P, op, base);
   if (!D.any_reg) {
     const float2 d = D.small ? D.pick(D.fixed) : D.Dg[D.fixed];
@@ -479,8 +486,8 @@ __device__ __forceinline__ void ew_diag(float2 (&v)[PER], const Prog& P, Op& op,
 
 // Products of phases on bit pairs (a CZ layer).  Pairs on thread / outer bits only multiply one
 // per-lane phase; pairs touching register bits multiply the elements whose e has those bits.
-template <int PER, int NT, class Prog, class Op>
-__device__ __forceinline__ void ew_pairs(float2 (&v)[PER], const Prog& P, Op& op, uint64_t base) {
+template <int PER, int NT, class Prog, class Op, class C>
+__device__ __forceinline__ void ew_pairs(C (&v)[PER], const Prog& P, Op& op, uint64_t base) {
   constexpr int TB = __builtin_ctz(NT);
   saux_t* pr = scalar_ptr(P.aux) + op.t[0];
   smat_t* ph = scalar_ptr(P.mats) + op.mat;
@@ -515,7 +522,7 @@ __device__ __forceinline__ void ew_pairs(float2 (&v)[PER], const Prog& P, Op& op
 #pragma unroll
     for (int e = 0; e < PER; ++e)
       if ((e & rneed) == rneed) {  // uniform test; the lane condition is a select
-        const float2 g = cmul(v[e], f);
+        const C g = cmul(v[e], f);
         v[e] = tc ? g : v[e];
       }
   }
@@ -535,8 +542,8 @@ __device__ __forceinline__ void ew_scale(float2 (&v)[PER], const Prog& P, Op& op
 // target m.  Local controls are tested on the group's base element (controls are never targets).
 // Without local controls (kCtl false) the groups are straight-line code: no per-group branch, so
 // results land in their own registers instead of being copied back at every branch join.
-template <int PER, int NT, int K, int R0, int R1, int R2, bool kCtl>
-__device__ __forceinline__ void reg_dense_k(float2 (&v)[PER], smat_t* M, int cm, int cv) {
+template <int PER, int NT, int K, int R0, int R1, int R2, bool kCtl, class MPtr>
+__device__ __forceinline__ void reg_dense_k(float2 (&v)[PER], MPtr M, int cm, int cv) {
   constexpr int D = 1 << K;
   constexpr int RS[3] = {R0, R1, R2};
   constexpr int TMASK = (1 << R0) | (K > 1 ? 1 << R1 : 0) | (K > 2 ? 1 << R2 : 0);
@@ -611,8 +618,8 @@ __device__ __forceinline__ void lane_swap(float& a, float& b) {
 }
 
 // 2x2 matrix M on lane bit T of every element.  Local controls (kCtl) are never the target bit.
-template <int PER, int NT, int T, bool kCtl>
-__device__ __forceinline__ void lane_reg_dense_k(float2 (&v)[PER], smat_t* M, int cm, int cv) {
+template <int PER, int NT, int T, bool kCtl, class MPtr>
+__device__ __forceinline__ void lane_reg_dense_k(float2 (&v)[PER], MPtr M, int cm, int cv) {
   const float2 m00 = ldm(M, 0), m01 = ldm(M, 1), m10 = ldm(M, 2), m11 = ldm(M, 3);
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));  // keeps the six bits' lane tests out of the registers between ops
@@ -812,8 +819,10 @@ __device__ __forceinline__ void tile_offsets(const int32_t* pos, uint64_t& off_l
                                              uint64_t (&off_hi)[TileShape<L>::PER]) {
   constexpr int TBL = TileShape<L>::TBL, PER = TileShape<L>::PER;
   off_lo = 0;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // the bits are formed again for the store, not kept (spilled) meanwhile
 #pragma unroll
-  for (int b = 0; b < TBL; ++b) off_lo |= (uint64_t)((threadIdx.x >> b) & 1) << pos[b];
+  for (int b = 0; b < TBL; ++b) off_lo |= (uint64_t)((tid >> b) & 1) << pos[b];
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
     uint64_t o = 0;
@@ -855,7 +864,20 @@ __device__ __forceinline__ void store_zero_tile(float2* __restrict__ psi, const 
 // basis >= 0 nothing is read: the tile starts as its part of the basis state |basis>.  Tiles whose
 // outer bits disagree with (zmask, zval) hold only zeros and store zeros; tiles whose outer bits
 // disagree with (wmask, wval) store nothing.
-template <int L, class Prog>
+struct RunProgram {  // the interpreter above
+  template <int PER, int NT, class Prog>
+  static __device__ __forceinline__ void run(float2 (&v)[PER], float2* tile, float2* mstage, const Prog& P,
+                                             uint64_t base, bool act) {
+    run_program<PER, NT>(v, tile, mstage, P, base, act);
+  }
+  template <int NT, class Prog>
+  static __device__ __forceinline__ void begin(const Prog& P, uint64_t, float2*) {
+    warm_program<NT>(P);
+  }
+};
+
+// Run: the interpreter (begin runs before the tile is loaded).
+template <int L, class Run = RunProgram, class Prog>
 __device__ __forceinline__ void pass_tile(float2* __restrict__ psi, const Prog& P, const int32_t* lpos,
                                           const int32_t* lpos_out, uint64_t base, float2* lds,
                                           int64_t basis = -1, uint64_t zmask = 0, uint64_t zval = 0,
@@ -871,7 +893,7 @@ __device__ __forceinline__ void pass_tile(float2* __restrict__ psi, const Prog& 
     store_zero_tile<L, PER, NT>(psi, lpos_out, base, act);
     return;
   }
-  warm_program<NT>(P);
+  Run::template begin<NT>(P, base, mstage);
   float2 v[PER];
   {
     uint64_t off_lo, off_hi[PER];
@@ -887,7 +909,7 @@ __device__ __forceinline__ void pass_tile(float2* __restrict__ psi, const Prog& 
       }
     }
   }
-  run_program<PER, NT>(v, tile, mstage, P, base, act);
+  Run::template run<PER, NT>(v, tile, mstage, P, base, act);
   {
     uint64_t off_lo, off_hi[PER];
     tile_offsets<L>(lpos_out, off_lo, off_hi);
