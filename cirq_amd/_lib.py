@@ -115,6 +115,7 @@ _SIGNATURES = {
     "cqs_expect_paulis_noalloc": ([_vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
     "cqs_apply_paulisum": ([_vp, _vp, _i32, _i32, _vp, _vp, _vp, _vp], ctypes.c_int),
     "cqs_norm2": ([_vp, _i32, _vp, _vp, _vp], ctypes.c_int),
+    "cqs_norm2_scaled": ([_vp, _i32, ctypes.c_float, _vp, _vp, _vp], ctypes.c_int),
     "cqs_inner": ([_vp, _vp, _i32, _vp, _vp, _vp], ctypes.c_int),
     "cqs_run_passes_specialized": ([_vp, _i32, ctypes.c_int64, _vp, _i32, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
     "cqs_adjoint_passes_specialized": ([_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _vp, ctypes.c_int64, _vp, _vp],

@@ -148,10 +148,11 @@ class Workspace:
         return self._buf
 
 
-def norm2(state: torch.Tensor, n_bits: int, ws: Workspace) -> float:
+def norm2(state: torch.Tensor, n_bits: int, ws: Workspace, scale: float = 1.0) -> float:
+    """Sum of |scale * amplitude|^2, each product rounded to complex64 as engine.scale stores it."""
     out = torch.zeros(2, dtype=torch.float64, device=state.device)
     w = ws.get(lib().cqs_expect_workspace_bytes(1))
-    check(lib().cqs_norm2(ptr(state), n_bits, ptr(out), ptr(w), stream_handle()), "cqs_norm2")
+    check(lib().cqs_norm2_scaled(ptr(state), n_bits, float(scale), ptr(out), ptr(w), stream_handle()), "cqs_norm2")
     return float(out[0].item())
 
 

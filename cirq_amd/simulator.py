@@ -965,7 +965,6 @@ class StateVectorTrialResult:
         self._ws = ws
         self._fsv = None
         self._scale = None
-        self._scaled = None
 
     def _renorm_factor(self) -> float:
         """1/norm when rescaling brings the total probability closer to 1, else 1
@@ -979,21 +978,20 @@ class StateVectorTrialResult:
             if abs(norm - 1) > eps:
                 warnings.warn(f"final state vector's norm={norm} is too far from 1, {abs(norm - 1)} > {eps}.")
             else:
-                t = self._state.clone()
-                engine.scale(t, n, 1.0 / norm)
-                n2b = engine.norm2(t, n, self._ws)
+                n2b = engine.norm2(self._state, n, self._ws, scale=1.0 / norm)
                 if abs(n2b - 1) < abs(n2 - 1):
                     self._scale = 1.0 / norm
-                    self._scaled = t
         return self._scale
 
     @property
     def final_state_vector(self) -> np.ndarray:
         """Copied to the host; renormalised only when that improves the total probability."""
         if self._fsv is None:
-            ret = self._scaled if self._renorm_factor() != 1.0 else self._state
+            ret = self._state
+            if self._renorm_factor() != 1.0:
+                ret = ret.clone()
+                engine.scale(ret, len(self._qubits), self._renorm_factor())
             self._fsv = ret.cpu().numpy()
-            self._scaled = None
         return self._fsv
 
     def state_vector(self, copy: bool = False) -> np.ndarray:

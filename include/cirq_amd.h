@@ -348,6 +348,10 @@ int cqs_inner(const void* a, const void* b, int32_t n_bits, double* out, void* w
  * cirq-core/cirq/qis/states.py:865-897 and cirq-core/cirq/sim/state_vector_simulator.py:131-146. */
 int cqs_norm2(const void* amps, int32_t n_bits, double* out, void* workspace, void* stream);
 
+/* out[0] = sum_i |scale amps[i]|^2 in FP64, every scale amps[i] rounded to FP32 as cqs_scale would
+ * store it: the norm of the scaled state without writing it. */
+int cqs_norm2_scaled(const void* amps, int32_t n_bits, float scale, double* out, void* workspace, void* stream);
+
 /* amps[i] = ((i & mask) == value) ? amps[i] * (re + i im) : 0: projection onto a measurement
  * outcome and renormalisation (cirq-core/cirq/sim/state_vector.py:235-322,
  * cirq-core/cirq/sim/density_matrix_utils.py:97-182 with the masks of both row and column bits). */

@@ -68,3 +68,17 @@ def test_density_matrix_terms(gpu, n, count):
         c = complex(cf[2 * t], cf[2 * t + 1])
         # 2^n entries of unit size in FP64
         assert abs(got[t] - c * np.sum(_signs(idx, zm[t]) * d)) < 2.0**-53 * 2**n * 8 * abs(c)
+
+
+@pytest.mark.parametrize("n", [0, 1, 5, 11, 12, 16])
+def test_norm_of_the_scaled_state_without_writing_it(gpu, n):
+    """engine.norm2 with a scale gives the bits of engine.scale followed by engine.norm2."""
+    from cirq_amd import engine
+
+    rng = np.random.RandomState(n)
+    st = torch.from_numpy((rng.randn(2**n) + 1j * rng.randn(2**n)).astype(np.complex64)).to(gpu)
+    ws = engine.Workspace(st.device)
+    for s in (1.0, 0.7310585, 1.0000001):
+        t = st.clone()
+        engine.scale(t, n, s)
+        assert engine.norm2(st, n, ws, scale=s) == engine.norm2(t, n, ws)
