@@ -13,6 +13,7 @@ import re
 from typing import Iterable
 
 
+@functools.lru_cache(maxsize=4096)
 def _pad_digits(text: str) -> str:
     """Natural-sort key of cirq.NamedQubit: runs of digits padded to 8 characters."""
     return re.sub(r"\d+", lambda m: m.group(0).rjust(8, "0"), text)
@@ -43,16 +44,8 @@ class Qid:
         return self._cmp_tuple() == other._cmp_tuple()
 
     def __hash__(self):
-        try:
-            return self._hash
-        except AttributeError:  # a qubit's key never changes; circuits look it up once per operation
-            self._hash = hash(self._cmp_tuple())
-            return self._hash
-
-    def __getstate__(self):
-        state = self.__dict__.copy()
-        state.pop("_hash", None)  # string hashes differ between processes
-        return state
+        # nothing is kept on the instance: a subclass may be a frozen dataclass, have slots or change
+        return hash(self._cmp_tuple())
 
 
 class LineQubit(Qid):
@@ -67,6 +60,11 @@ class LineQubit(Qid):
 
     def _comparison_key(self):
         return (self._x,)
+
+    def __hash__(self):
+        if type(self) is not LineQubit:  # a subclass may have a key of its own
+            return super().__hash__()
+        return hash(("LineQubit", (self._x,)))  # of _cmp_tuple, without its calls: every dict lookup of an op asks
 
     @staticmethod
     def range(*args) -> list["LineQubit"]:
@@ -99,6 +97,11 @@ class GridQubit(Qid):
 
     def _comparison_key(self):
         return (self._row, self._col)
+
+    def __hash__(self):
+        if type(self) is not GridQubit:  # a subclass may have a key of its own
+            return super().__hash__()
+        return hash(("GridQubit", (self._row, self._col)))  # of _cmp_tuple, without its calls: every dict lookup of an op asks
 
     @staticmethod
     def rect(rows: int, cols: int, top: int = 0, left: int = 0) -> list["GridQubit"]:
