@@ -239,6 +239,18 @@ class _QubitsOnly:
         self.n_bits = 2 * self.n if dm else self.n
 
 
+def _observable_terms(observables, qmap, n: int):
+    """(pauli_masks of every term, index of the observable each belongs to).  KeyError for a term on
+    a qubit outside the circuit; terms of coefficient 0 are dropped wherever they act."""
+    terms, owner = [], []
+    for oi, o in enumerate(observables):
+        # a string that is not zero is its own only term; sums merge theirs and drop zeros
+        for t in (o,) if type(o) is PauliString and o.coefficient != 0 else PauliSum.wrap(o):
+            terms.append(pauli_masks(t, qmap, n))
+            owner.append(oi)
+    return terms, np.array(owner, dtype=np.int64)
+
+
 class _SimulatorBase:
     _dm = False
 
@@ -880,13 +892,7 @@ class _SimulatorBase:
         qubits = QubitOrder.as_qubit_order(qubit_order).order_for(circuit.all_qubits())
         qmap = {q: i for i, q in enumerate(qubits)}
         n = len(qubits)
-        terms, owner = [], []
-        for oi, o in enumerate(observables):
-            # one string is its own only term; sums merge theirs
-            for t in (o,) if type(o) is PauliString else PauliSum.wrap(o):
-                terms.append(pauli_masks(t, qmap, n))  # KeyError for a qubit outside the circuit
-                owner.append(oi)
-        owner = np.array(owner, dtype=np.int64)
+        terms, owner = _observable_terms(observables, qmap, n)
 
         def values(st):
             vals = engine.expect_terms(st, n, self._dm, terms, self._ws).cpu().numpy()

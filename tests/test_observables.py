@@ -155,3 +155,19 @@ def test_errors():
                                       num_samples=10)
     with pytest.raises(ValueError):
         obs.sample_expectation_values(OracleSampler(), c, [1j * cirq.Z(q[0])], num_samples=10)
+
+
+def test_zero_strings_act_on_any_qubit():
+    """A string of coefficient 0 has no term, alone or in a sum, also on a qubit outside the circuit; others there
+    are refused."""
+    from cirq_amd.simulator import _observable_terms
+
+    a, b = cirq.LineQubit.range(2)
+    qmap = {a: 0}
+    z = cirq.Z(a) * 2.0
+    for zero in (0 * cirq.Z(b), cirq.PauliString(cirq.Z(b), coefficient=0), cirq.PauliSum.wrap(0 * cirq.Z(b)), 0 * cirq.Z(a)):
+        terms, owner = _observable_terms([zero, z], qmap, 1)
+        assert terms == [(0, 1, 2.0)] and list(owner) == [1]
+    for outside in (cirq.Z(b) * 1.0, cirq.Z(a) * 1.0 + cirq.X(b), cirq.X(b)):
+        with pytest.raises(KeyError):
+            _observable_terms([outside], qmap, 1)
