@@ -487,12 +487,14 @@ int cqs_permuted_probs(const void* amps, int32_t n_qubits, int32_t is_dm, const 
 /*
  * Index -> big-endian digits: out[r*m + k] = bit (m-1-k) of index[r]
  * (cirq-core/cirq/value/digits.py:125-170 as used by cirq-core/cirq/sim/state_vector.py:228-232).
+ * DEVICE arrays; asynchronous on the stream.
  */
 int cqs_indices_to_bits(const int64_t* index, int64_t reps, int32_t m, uint8_t* out, void* stream);
 
 /*
  * The same digits into chosen columns of rows of `width` bytes: out[r*width + columns[k]] = bit
- * (m-1-k) of index[r] (columns: HOST, m entries in [0, width)); the other columns are left alone.
+ * (m-1-k) of index[r]; the other columns are left alone.  index and out are DEVICE arrays, columns a
+ * HOST array of m entries in [0, width); asynchronous on the stream.
  */
 int cqs_indices_to_columns(const int64_t* index, int64_t reps, int32_t m, const int32_t* columns, int32_t width,
                            uint8_t* out, void* stream);
