@@ -8,7 +8,7 @@
 // any two ops, so a gate is undone by one op instead of one per state.
 //
 // GRAD sums are sums of the products conj(phi_i) psi_j weighted by G's entries.  The products are formed
-// in FP32 and summed in FP64, only those whose entry of G is not zero (a uniform test): a
+// and summed in FP64, only those whose entry of G is not zero (a uniform test): a
 // rotation about X, Y or Z has two real numbers in its generator.  Diagonal ops on both states leave
 // conj(phi_j) psi_j as it is, so a run of them forms the products once for all its GRAD ops and
 // multiplies the states once by the run's accumulated phases (DiagRun).  The reverse passes are
@@ -25,10 +25,11 @@ constexpr int kSelBoth = 0, kSelPsi = 1, kSelPhi = 2;
 __device__ __forceinline__ int op_kind(sop_t& op) { return op.kind & 0xff; }
 __device__ __forceinline__ int op_sel(sop_t& op) { return (op.kind >> 8) & 3; }
 
-// conj(f) x, its real or its imaginary part, in FP32 as the states (summed in FP64).
+// s + conj(f) x, its real or its imaginary part, in FP64: the products of two FP32 values are exact there.
 template <bool kImag>
-__device__ __forceinline__ float overlap(float2 f, float2 x) {
-  return kImag ? fmaf(f.x, x.y, -f.y * x.x) : fmaf(f.x, x.x, f.y * x.y);
+__device__ __forceinline__ double add_overlap(double s, float2 f, float2 x) {
+  const double fr = f.x, fi = f.y, xr = x.x, xi = x.y;
+  return kImag ? fma(fr, xi, fma(-fi, xr, s)) : fma(fr, xr, fma(fi, xi, s));
 }
 
 // 2 Re sum over pairs (m, n) of one bit of conj(f) M x, for a 2x2 M: the products that M's nonzero
@@ -45,13 +46,13 @@ __device__ __forceinline__ double grad_pairs(int pairs, X x, F f, MPtr M) {
       if (m.x != 0.f) {
         double s = 0.0;
 #pragma unroll
-        for (int i = 0; i < pairs; ++i) s += (double)overlap<false>(f(i, r), x(i, c));
+        for (int i = 0; i < pairs; ++i) s = add_overlap<false>(s, f(i, r), x(i, c));
         g = fma((double)m.x, s, g);
       }
       if (m.y != 0.f) {
         double s = 0.0;
 #pragma unroll
-        for (int i = 0; i < pairs; ++i) s += (double)overlap<true>(f(i, r), x(i, c));
+        for (int i = 0; i < pairs; ++i) s = add_overlap<true>(s, f(i, r), x(i, c));
         g = fma(-(double)m.y, s, g);
       }
     }
@@ -211,13 +212,13 @@ __device__ __forceinline__ double grad_lane1(const float2 (&x)[PER], const float
   if (m00.x != 0.f || m11.x != 0.f) {
     double s = 0.0;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) s += (double)overlap<false>(f[e], x[e]);
+    for (int e = 0; e < PER; ++e) s = add_overlap<false>(s, f[e], x[e]);
     g = fma((double)d.x, s, g);
   }
   if (m00.y != 0.f || m11.y != 0.f) {
     double s = 0.0;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) s += (double)overlap<true>(f[e], x[e]);
+    for (int e = 0; e < PER; ++e) s = add_overlap<true>(s, f[e], x[e]);
     g = fma(-(double)d.y, s, g);
   }
   const bool re = m01.x != 0.f || m10.x != 0.f, im = m01.y != 0.f || m10.y != 0.f;
@@ -226,8 +227,8 @@ __device__ __forceinline__ double grad_lane1(const float2 (&x)[PER], const float
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       const float2 p = make_float2(lane_xor<T>(x[e].x), lane_xor<T>(x[e].y));
-      if (re) sr += (double)overlap<false>(f[e], p);
-      if (im) si += (double)overlap<true>(f[e], p);
+      if (re) sr = add_overlap<false>(sr, f[e], p);
+      if (im) si = add_overlap<true>(si, f[e], p);
     }
     g = fma((double)o.x, sr, g);
     g = fma(-(double)o.y, si, g);
@@ -277,7 +278,7 @@ __device__ __forceinline__ double grad_reg_dense(const float2 (&x)[PER], const f
 // out (QAOA gradient off by 7e-6 instead of 2e-6).
 template <int PER, int NT>
 struct DiagRun {
-  float w[PER];
+  double w[PER];
   double2 ph[PER];
   bool have_w = false, have_ph = false;
 
@@ -288,7 +289,7 @@ struct DiagRun {
                                          uint64_t base) {
     if (!have_w) {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) w[e] = overlap<true>(f[e], x[e]);
+      for (int e = 0; e < PER; ++e) w[e] = add_overlap<true>(0.0, f[e], x[e]);
       have_w = true;
     }
     const DiagTable<PER, NT, Prog> D(P, op, base);
@@ -296,18 +297,18 @@ struct DiagRun {
     if (!D.any_reg) {
       const float2 d = D.small ? D.pick(D.fixed) : D.Dg[D.fixed];
 #pragma unroll
-      for (int e = 0; e < PER; ++e) acc += (double)w[e];
+      for (int e = 0; e < PER; ++e) acc += w[e];
       acc *= -(double)d.y;
     } else if (D.small) {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) acc = fma(-(double)D.pick(D.index(e)).y, (double)w[e], acc);
+      for (int e = 0; e < PER; ++e) acc = fma(-(double)D.pick(D.index(e)).y, w[e], acc);
     } else {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) acc = fma(-(double)D.Dg[D.index(e)].y, (double)w[e], acc);
+      for (int e = 0; e < PER; ++e) acc = fma(-(double)D.Dg[D.index(e)].y, w[e], acc);
     }
     if (!D.small || D.d0.x != 0.f || D.d1.x != 0.f || D.d2.x != 0.f || D.d3.x != 0.f) {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) acc = fma((double)D.at(e).x, (double)overlap<false>(f[e], x[e]), acc);
+      for (int e = 0; e < PER; ++e) acc = fma((double)D.at(e).x, add_overlap<false>(0.0, f[e], x[e]), acc);
     }
     return 2.0 * acc;
   }

@@ -308,7 +308,7 @@ __device__ __forceinline__ void adjoint_staged(float2 (&va)[PER], float2 (&vb)[P
     if (cls >= kElem) {
       // a run of diagonal ops on both states, which leave the products conj(f) x as they are: formed once
       // (DiagRun also gathers the phases, in FP64: slower here, 2.48 against 1.85 ms for the 20-qubit ansatz)
-      float w[PER];
+      double w[PER];
       double total = 0.0;
       bool have_w = false;
       do {
@@ -316,8 +316,8 @@ __device__ __forceinline__ void adjoint_staged(float2 (&va)[PER], float2 (&vb)[P
           if (!have_w) {
 #pragma unroll
             for (int e = 0; e < PER; ++e) {
-              w[e] = overlap<true>(vb[e], va[e]);
-              total += (double)w[e];
+              w[e] = add_overlap<true>(0.0, vb[e], va[e]);
+              total += w[e];
             }
             have_w = true;
           }
@@ -333,7 +333,7 @@ __device__ __forceinline__ void adjoint_staged(float2 (&va)[PER], float2 (&vb)[P
             double s = 0.0;  // elements with the register bit set
 #pragma unroll
             for (int e = 0; e < PER; ++e)
-              if (e & bit) s += (double)w[e];
+              if (e & bit) s += w[e];
             g = -2.0 * fma((double)hi.y, s, (double)lo.y * (total - s));
           }
           write_wave_partial<NT>(act ? g : 0.0, partial, stride, tile, rec_word(r, 2));
