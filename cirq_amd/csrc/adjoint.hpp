@@ -10,8 +10,7 @@
 // GRAD sums are sums of the products conj(phi_i) psi_j weighted by G's entries.  The products are formed
 // and summed in FP64, only those whose entry of G is not zero (a uniform test): a
 // rotation about X, Y or Z has two real numbers in its generator.  Diagonal ops on both states leave
-// conj(phi_j) psi_j as it is, so a run of them forms the products once for all its GRAD ops and
-// multiplies the states once by the run's accumulated phases (DiagRun).  The reverse passes are
+// conj(phi_j) psi_j as it is, so a run of them forms the products once for all its GRAD ops (specialised and decoded passes).  The reverse passes are
 // bound by VALU work and latency: a gradient of 24-node QAOA, 8 rounds (36 ZZ and 24 X rotations each), takes
 // 7.0 ms against 8.5 with dU, psi-only and phi-only ops; of the 20-qubit ansatz, 400 rotations, 2.24 against 2.74.
 #pragma once
@@ -271,71 +270,57 @@ __device__ __forceinline__ double grad_reg_dense(const float2 (&x)[PER], const f
 #undef CQS_G3
 }
 
-// A run of diagonal ops on both states (x: psi, f: phi): the products w_j = Im conj(f_j) x_j, formed
-// at the run's first GRAD_DIAG, serve all of them, and the run's phases are multiplied into the
-// states once, when it ends.  The phases' product is kept in FP64: rounded to FP32 after every op, elements
-// with equal phases would all drift alike, and the run's rounding errors would add up instead of averaging
-// out (QAOA gradient off by 7e-6 instead of 2e-6).
-template <int PER, int NT>
-struct DiagRun {
-  double w[PER];
-  double2 ph[PER];
-  bool have_w = false, have_ph = false;
+// Diagonal gradients weight the products w_e = Im conj(f_e) x_e of this thread's elements (x: psi, f: phi).
+// Diagonal ops of unit modulus on both states leave the products as they are, so specialised passes form them once for a
+// run of such ops.  They are plain arrays of the calling kernel: as members of an object with flags for what was formed
+// they went to scratch memory (208 bytes per lane; reverse passes of the 20-qubit ansatz 0.85 ms against 0.52).
+template <int PER>
+__device__ __forceinline__ void diag_products(double (&w)[PER], const float2 (&x)[PER], const float2 (&f)[PER]) {
+#pragma unroll
+  for (int e = 0; e < PER; ++e) w[e] = add_overlap<true>(0.0, f[e], x[e]);
+}
 
-  // 2 Re sum conj(f_j) d(j) x_j for a diagonal d.  A generator's entries are imaginary: only w is
-  // needed; a nonzero real part (a uniform test for tables of up to 4 entries) adds its products.
-  template <class Prog, class Op>
-  __device__ __forceinline__ double grad(const float2 (&x)[PER], const float2 (&f)[PER], const Prog& P, Op& op,
-                                         uint64_t base) {
-    if (!have_w) {
+// 2 Re sum conj(f_e) d(e) x_e for a diagonal d and w(e) the products above.  A generator's entries are imaginary: only
+// w is needed; a nonzero real part (a uniform test for tables of up to 4 entries) adds its products.
+template <int PER, int NT, class W, class Prog, class Op>
+__device__ __forceinline__ double grad_diag(W w, const float2 (&x)[PER], const float2 (&f)[PER], const Prog& P, Op& op,
+                                            uint64_t base) {
+  const DiagTable<PER, NT, Prog> D(P, op, base);
+  double acc = 0.0;
+  if (!D.any_reg) {
+    const float2 d = D.small ? D.pick(D.fixed) : D.Dg[D.fixed];
 #pragma unroll
-      for (int e = 0; e < PER; ++e) w[e] = add_overlap<true>(0.0, f[e], x[e]);
-      have_w = true;
-    }
-    const DiagTable<PER, NT, Prog> D(P, op, base);
-    double acc = 0.0;
-    if (!D.any_reg) {
-      const float2 d = D.small ? D.pick(D.fixed) : D.Dg[D.fixed];
+    for (int e = 0; e < PER; ++e) acc += w(e);
+    acc *= -(double)d.y;
+  } else if (D.small) {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) acc += w[e];
-      acc *= -(double)d.y;
-    } else if (D.small) {
+    for (int e = 0; e < PER; ++e) acc = fma(-(double)D.pick(D.index(e)).y, w(e), acc);
+  } else {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) acc = fma(-(double)D.pick(D.index(e)).y, w[e], acc);
-    } else {
-#pragma unroll
-      for (int e = 0; e < PER; ++e) acc = fma(-(double)D.Dg[D.index(e)].y, w[e], acc);
-    }
-    if (!D.small || D.d0.x != 0.f || D.d1.x != 0.f || D.d2.x != 0.f || D.d3.x != 0.f) {
-#pragma unroll
-      for (int e = 0; e < PER; ++e) acc = fma((double)D.at(e).x, add_overlap<false>(0.0, f[e], x[e]), acc);
-    }
-    return 2.0 * acc;
+    for (int e = 0; e < PER; ++e) acc = fma(-(double)D.Dg[D.index(e)].y, w(e), acc);
   }
-  // The run's phases, to be multiplied by a diagonal op's (ew_diag, ew_pairs).
-  __device__ __forceinline__ double2 (&phases())[PER] {
-    if (!have_ph) {
+  if (!D.small || D.d0.x != 0.f || D.d1.x != 0.f || D.d2.x != 0.f || D.d3.x != 0.f) {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) ph[e] = make_double2(1.0, 0.0);
-      have_ph = true;
-    }
-    return ph;
+    for (int e = 0; e < PER; ++e) acc = fma((double)D.at(e).x, add_overlap<false>(0.0, f[e], x[e]), acc);
   }
-  __device__ __forceinline__ void finish(float2 (&x)[PER], float2 (&f)[PER]) {
-    if (!have_ph) return;
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const float2 p = make_float2((float)ph[e].x, (float)ph[e].y);
-      x[e] = cmul(x[e], p);
-      f[e] = cmul(f[e], p);
-    }
-  }
-};
+  return 2.0 * acc;
+}
 
-// Whether a diagonal op belongs to a DiagRun: GRAD_DIAG, and DIAG or PAIRPHASE on both states.
-__device__ __forceinline__ bool in_diag_run(sop_t& op) {
-  const int kind = op_kind(op);
-  return kind == CQS_OP_GRAD_DIAG || ((kind == CQS_OP_DIAG || kind == CQS_OP_PAIRPHASE) && op_sel(op) == kSelBoth);
+// Phases that all of a thread's elements share (no register bit among an op's bits), gathered over a run in FP64 and
+// multiplied into both states once; phases that differ between elements are multiplied op by op.
+template <int PER, int NT, class Prog, class Op>
+__device__ __forceinline__ void gather_diag(double2& ph, const Prog& P, Op& op, uint64_t base) {
+  const DiagTable<PER, NT, Prog> D(P, op, base);
+  ph = cmul(ph, D.small ? D.pick(D.fixed) : D.Dg[D.fixed]);
+}
+template <int PER>
+__device__ __forceinline__ void apply_phase(float2 (&x)[PER], float2 (&f)[PER], double2 ph) {
+  const float2 p = make_float2((float)ph.x, (float)ph.y);
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    x[e] = cmul(x[e], p);
+    f[e] = cmul(f[e], p);
+  }
 }
 
 // Every wave writes its own partial of a GRAD op: partial[slot * stride + tile * NW + wave] (a
@@ -352,8 +337,7 @@ __device__ __forceinline__ void write_wave_partial(double g, double* __restrict_
 // per-slot partial entries).
 __host__ __device__ constexpr int adjoint_waves(int L) { return (L <= 12 ? 256 : (1 << L) / 16) / 64; }
 
-// One op of a register phase on this thread's elements of both states (a diagonal gradient alone:
-// adjoint_tile keeps runs together).
+// One op of a register phase on this thread's elements of both states.
 template <int PER, int NT, class Prog>
 __device__ __forceinline__ void adjoint_register_op(float2 (&va)[PER], float2 (&vb)[PER], const Prog& P, sop_t& op,
                                                     uint64_t base, bool act, double* __restrict__ partial,
@@ -361,9 +345,9 @@ __device__ __forceinline__ void adjoint_register_op(float2 (&va)[PER], float2 (&
   const int kind = op_kind(op), sel = op_sel(op);
   const bool ok = outer_controls_ok(op, base);
   if (kind == CQS_OP_GRAD_DIAG) {
-    DiagRun<PER, NT> run;
     double g = 0.0;
-    if (ok && act) g = run.grad(va, vb, P, op, base);
+    if (ok && act)
+      g = grad_diag<PER, NT>([&](int e) { return add_overlap<true>(0.0, vb[e], va[e]); }, va, vb, P, op, base);
     write_wave_partial<NT>(g, partial, stride, tile, op.slot);
     return;
   }
@@ -477,31 +461,8 @@ __device__ __forceinline__ void RunAdjoint::run(float2 (&va)[PER], float2 (&vb)[
   int i = 0;
   for (;;) {
     // register phase
-    for (; i < P.op_count && !adj_mixing<PER, NT>(scalar_ptr(P.ops)[i]); ++i) {
-      sop_t& op = scalar_ptr(P.ops)[i];
-      if (in_diag_run(op)) {
-        DiagRun<PER, NT> run;
-        for (;; ++i) {
-          sop_t& d = scalar_ptr(P.ops)[i];
-          const int dk = op_kind(d);
-          const bool dok = outer_controls_ok(d, base);
-          if (dk == CQS_OP_GRAD_DIAG) {
-            double g = 0.0;
-            if (dok && act) g = run.grad(va, vb, P, d, base);
-            write_wave_partial<NT>(g, partial, stride, tile, d.slot);
-          } else if (dok) {
-            if (dk == CQS_OP_DIAG)
-              ew_diag<PER, NT>(run.phases(), P, d, base);
-            else
-              ew_pairs<PER, NT>(run.phases(), P, d, base);
-          }
-          if (i + 1 >= P.op_count || !in_diag_run(scalar_ptr(P.ops)[i + 1])) break;
-        }
-        run.finish(va, vb);
-        continue;
-      }
-      adjoint_register_op<PER, NT>(va, vb, P, op, base, act, partial, stride, tile);
-    }
+    for (; i < P.op_count && !adj_mixing<PER, NT>(scalar_ptr(P.ops)[i]); ++i)
+      adjoint_register_op<PER, NT>(va, vb, P, scalar_ptr(P.ops)[i], base, act, partial, stride, tile);
     if (i >= P.op_count) break;
     // LDS phase: both tiles out of registers, then every consecutive op that mixes threads
     regs_to_tile<PER, NT>(va, tA, act);

@@ -466,8 +466,8 @@ struct DiagTable {
   __device__ __forceinline__ float2 at(int e) const { return small ? pick(index(e)) : Dg[index(e)]; }
 };
 
-template <int PER, int NT, class Prog, class Op, class C>
-__device__ __forceinline__ void ew_diag(C (&v)[PER], const Prog& P, Op& op, uint64_t base) {
+template <int PER, int NT, class Prog, class Op>
+__device__ __forceinline__ void ew_diag(float2 (&v)[PER], const Prog& P, Op& op, uint64_t base) {
   const DiagTable<PER, NT, Prog> D(P, op, base);
   if (!D.any_reg) {
     const float2 d = D.small ? D.pick(D.fixed) : D.Dg[D.fixed];
@@ -486,8 +486,8 @@ __device__ __forceinline__ void ew_diag(C (&v)[PER], const Prog& P, Op& op, uint
 
 // Products of phases on bit pairs (a CZ layer).  Pairs on thread / outer bits only multiply one
 // per-lane phase; pairs touching register bits multiply the elements whose e has those bits.
-template <int PER, int NT, class Prog, class Op, class C>
-__device__ __forceinline__ void ew_pairs(C (&v)[PER], const Prog& P, Op& op, uint64_t base) {
+template <int PER, int NT, class Prog, class Op>
+__device__ __forceinline__ void ew_pairs(float2 (&v)[PER], const Prog& P, Op& op, uint64_t base) {
   constexpr int TB = __builtin_ctz(NT);
   saux_t* pr = scalar_ptr(P.aux) + op.t[0];
   smat_t* ph = scalar_ptr(P.mats) + op.mat;
@@ -522,7 +522,7 @@ __device__ __forceinline__ void ew_pairs(C (&v)[PER], const Prog& P, Op& op, uin
 #pragma unroll
     for (int e = 0; e < PER; ++e)
       if ((e & rneed) == rneed) {  // uniform test; the lane condition is a select
-        const C g = cmul(v[e], f);
+        const float2 g = cmul(v[e], f);
         v[e] = tc ? g : v[e];
       }
   }

@@ -32,6 +32,7 @@ from pathlib import Path
 import numpy as np
 
 from . import _build, _lib
+from .tape import OUTER
 
 CSRC = Path(__file__).resolve().parent / "csrc"
 CACHE_DIR = Path(os.environ.get("CIRQ_AMD_SPECIALIZE_CACHE", Path(__file__).resolve().parent / "_specialized"))
@@ -250,7 +251,7 @@ def _adj_mixing(op, nt: int, per: int) -> bool:
 
 
 def _in_diag_run(op) -> bool:
-    """adjoint.hpp in_diag_run: GRAD_DIAG, and DIAG or PAIRPHASE on both states."""
+    """Whether an op belongs to a run of diagonal ops: GRAD_DIAG, and DIAG or PAIRPHASE on both states."""
     kind, sel = int(op["kind"]) & 0xFF, (int(op["kind"]) >> 8) & 3
     return kind == _lib.OP_GRAD_DIAG or (kind in (_OP_DIAG, _OP_PAIR) and sel == 0)
 
@@ -264,12 +265,53 @@ def _guard_cond(op) -> str:
     return f"(base & 0x{mask:x}ull) == 0x{val:x}ull"
 
 
-def adjoint_pass_source(index: int, ps, ops: np.ndarray) -> str:
+def _diag_run_source(index: int, ops, begin: int, end: int, tb: int) -> str:
+    """A run of diagonal ops: its gradient ops weight products formed once (adjoint.hpp diag_products).  Phases
+    without register bits are gathered (gather_diag) where there are several; what is formed when is
+    known here, so the kernel holds plain arrays and no flags."""
+
+    def kind(j):
+        return int(ops[j]["kind"]) & 0xFF
+
+    def shared(j):  # all of a thread's elements see the same phase
+        return kind(j) == _OP_DIAG and all(int(x) < tb or int(x) >= OUTER for x in ops[j]["t"][: int(ops[j]["k"])])
+
+    gather = sum(shared(j) for j in range(begin, end)) > 1
+    out = ["  {"]
+    if gather:
+        out.append("    double2 ph = make_double2(1.0, 0.0);")
+    formed = False
+    for j in range(begin, end):
+        ref, cond = f"kA{index}_{j}", _guard_cond(ops[j])
+        if kind(j) == _lib.OP_GRAD_DIAG:
+            if not formed:
+                out.append("    double w[PER];\n    diag_products<PER>(w, va, vb);")
+                formed = True
+            out.append(f"    {{\n      double g = 0.0;\n      if (({cond}) && act) g = grad_diag<PER, NT>([&](int e) {{ return w[e]; }}, "
+                       f"va, vb, P, {ref}, base);\n"
+                       f"      write_wave_partial<NT>(g, partial, stride, tile, {int(ops[j]['slot'])});\n    }}")
+            continue
+        guard = "" if cond == "true" else f"if ({cond}) "
+        if gather and shared(j):
+            out.append(f"    {guard}gather_diag<PER, NT>(ph, P, {ref}, base);")
+        else:
+            call = "ew_diag" if kind(j) == _OP_DIAG else "ew_pairs"
+            out += [f"    {guard}{call}<PER, NT>({st}, P, {ref}, base);" for st in ("va", "vb")]
+    if gather:
+        out.append("    apply_phase<PER>(va, vb, ph);")
+    return "\n".join(out + ["  }"])
+
+
+def adjoint_pass_source(index: int, ps, ops: np.ndarray, n_bits: int) -> str:
     """HIP source of one reverse-sweep pass as `extern "C" __global__ void k_aspec_<index>(float2*
     psi, float2* phi, TileProg, double* partial, int64_t stride)`, the same steps as adjoint.hpp
-    adjoint_tile for this pass's ops."""
+    adjoint_tile for this pass's ops, on states of n_bits bits."""
     L = int(ps["L"])
     nt, per = _shape(L)
+    # The two tiles of up to 2^11 amplitudes leave room in LDS for four workgroups per CU, i.e. four waves per SIMD:
+    # registers are held to 128 where there are tiles enough for them (24-bit states: a noisy gradient's reverse passes
+    # 12.3 ms against 13.4), and not where each CU has at most two workgroups (20 bits: 0.52 against 0.53 ms).
+    waves = 4 if L <= 11 and n_bits - L > 9 else 2
     tb = nt.bit_length() - 1
     first, count = int(ps["op_begin"]), int(ps["op_count"])
     consts = "".join(_op_constant(f"kA{index}_{j}", ops[first + j]) for j in range(count))
@@ -281,20 +323,11 @@ def adjoint_pass_source(index: int, ps, ops: np.ndarray) -> str:
         kind, sel = int(op["kind"]) & 0xFF, (int(op["kind"]) >> 8) & 3
         ref = f"kA{index}_{j}"
         if _in_diag_run(op):
-            run = ["  {\n    DiagRun<PER, NT> run;"]
-            while j < count and _in_diag_run(ops[first + j]):
-                op = ops[first + j]
-                kind, ref, cond = int(op["kind"]) & 0xFF, f"kA{index}_{j}", _guard_cond(op)
-                if kind == _lib.OP_GRAD_DIAG:
-                    run.append(f"    {{\n      double g = 0.0;\n      if (({cond}) && act) g = run.grad(va, vb, P, {ref}, base);\n"
-                               f"      write_wave_partial<NT>(g, partial, stride, tile, {int(op['slot'])});\n    }}")
-                else:
-                    guard = "" if cond == "true" else f"if ({cond}) "
-                    call = "ew_diag" if kind == _OP_DIAG else "ew_pairs"
-                    run.append(f"    {guard}{call}<PER, NT>(run.phases(), P, {ref}, base);")
-                j += 1
-            run.append("    run.finish(va, vb);\n  }")
-            body.append("\n".join(run))
+            end = j
+            while end < count and _in_diag_run(ops[first + end]):
+                end += 1
+            body.append(_diag_run_source(index, ops[first : first + count], j, end, tb))
+            j = end
             continue
         if not _adj_mixing(op, nt, per):
             cond = _guard_cond(op)
@@ -351,7 +384,7 @@ def adjoint_pass_source(index: int, ps, ops: np.ndarray) -> str:
         body.append("  __syncthreads();\n  tile_to_regs<PER, NT>(va, tA, act);\n  tile_to_regs<PER, NT>(vb, tB, act);")
     lines = "\n".join(body)
     return consts + f"""
-extern "C" __global__ __launch_bounds__({nt}) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_aspec_{index}(
+extern "C" __global__ __launch_bounds__({nt}) __attribute__((amdgpu_waves_per_eu({waves}, 8))) void k_aspec_{index}(
     float2* __restrict__ psi, float2* __restrict__ phi, TileProg P, double* __restrict__ partial, int64_t stride) {{
   constexpr int L = {L}, NT = {nt}, PER = {per};
   extern __shared__ float2 lds[];
@@ -401,8 +434,10 @@ def program_sources(packed, adjoint: bool = False) -> list[str]:
     translation unit."""
     head = f'#include "{CSRC / ("adjoint.hpp" if adjoint else "tile.hpp")}"\nusing namespace cqs;\n'
     ops = packed.ops_arr
-    gen = adjoint_pass_source if adjoint else pass_source
-    kernels = [gen(i, ps, ops) for i, ps in enumerate(packed.pass_arr)]
+    if adjoint:
+        kernels = [adjoint_pass_source(i, ps, ops, packed.n_bits) for i, ps in enumerate(packed.pass_arr)]
+    else:
+        kernels = [pass_source(i, ps, ops) for i, ps in enumerate(packed.pass_arr)]
     per = 1 if adjoint else KERNELS_PER_FILE  # reverse-sweep kernels are several times larger
     return [head + "".join(kernels[i : i + per]) for i in range(0, len(kernels), per)]
 
