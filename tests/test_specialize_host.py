@@ -3,6 +3,7 @@ interpreter's dispatch for every op kind, and a small program compiles and expos
 handle per pass (no GPU needed; the GPU parity is tests/test_gpu_specialize.py)."""
 
 import numpy as np
+import pytest
 
 from cirq_amd import _lib, generators, specialize, tape
 from tests.test_host import _random_circuit
@@ -80,3 +81,26 @@ def test_reverse_sweep_sources_write_one_partial_per_gradient_slot():
     kinds = prog.rev.ops_arr["kind"][: prog.rev.n_ops] & 0xFF
     grads = int(((kinds == _lib.OP_GRAD_DIAG) | (kinds == _lib.OP_GRAD_DENSE)).sum())
     assert grads == prog.n_slots
+
+
+@pytest.mark.parametrize("ops,reads,writes", [
+    ([("dense", (9, 10), 2)], {"phi"}, {"phi"}),                      # a channel's adjoint, in registers
+    ([("dense", (0, 7), 2)], {"phi"}, {"phi"}),                       # through LDS
+    ([("grad_diag", (1,), 0)], {"psi", "phi"}, set()),                # gradients alone write neither state
+    ([("grad_dense", (7,), 0), ("dense", (2,), 1)], {"psi", "phi"}, {"psi"}),
+    ([("dense", (0, 7), 2), ("dense", (3,), 0)], {"psi", "phi"}, {"psi", "phi"}),
+])
+def test_reverse_pass_moves_only_the_states_its_ops_touch(ops, reads, writes):
+    def op(kind, targets, sel):
+        d = 2 ** len(targets)
+        mat = np.ones(d) if kind == "grad_diag" else np.eye(d)
+        return tape.LOp(kind, targets, mat, (), None, sel, 0 if kind.startswith("grad") else -1)
+
+    packed = tape.PackedProgram([tape.Pass(11, tuple(range(11)), [op(*o) for o in ops])], 12)
+    (text,) = specialize.program_sources(packed, adjoint=True)
+    body = text[text.index("warm_program") :]
+    assert {s for s in ("psi", "phi") if f"= {s}[" in body} == reads
+    assert {s for s in ("psi", "phi") if f" {s}[base + off_lo + off_hi[e]] =" in body} == writes
+    through = ops[0][0] == "dense" and 7 in ops[0][1]
+    assert ("regs_to_tile<PER, NT>(vb, tB" in body) == (through or ops[0][0] == "grad_dense")
+    assert not through or "regs_to_tile<PER, NT>(va, tA" not in body
