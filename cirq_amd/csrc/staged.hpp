@@ -40,8 +40,12 @@ enum StagedClass : int {
   kGradElemReg = 56,
 };
 
-// Decodes op i of the pass for the tile at `base`.  TB: thread bits.
-template <int TB, class Prog>
+// |d| = 1 as far as FP32 holds it.
+__device__ __forceinline__ bool unit_modulus(float2 d) { return fabsf(fmaf(d.x, d.x, d.y * d.y) - 1.f) < 1e-6f; }
+
+// Decodes op i of the pass for the tile at `base`.  TB: thread bits.  In reverse passes the elementwise classes are ops of
+// unit modulus on both states, which leave conj(phi) psi as it is; others end a run of diagonal ops (kGeneric).
+template <int TB, bool kReverse, class Prog>
 __device__ __forceinline__ void decode_op(const Prog& P, int i, uint64_t base, int* r) {
   struct Words {
     int w[16];
@@ -84,7 +88,7 @@ __device__ __forceinline__ void decode_op(const Prog& P, int i, uint64_t base, i
   } else if (kind == CQS_OP_SCALE && sel == 0) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) e[q] = P.mats[mat];
-    cls = kElem;
+    cls = kReverse && !unit_modulus(e[0]) ? kGeneric : kElem;
   } else if ((kind == CQS_OP_DIAG || kind == CQS_OP_GRAD_DIAG) && k <= 2 && sel == 0) {
     // entry index bit 0 <- s0, bit 1 <- s1: a tile bit, or -1 for none
     int s0 = t0, s1 = k == 2 ? t1 : -1;
@@ -117,7 +121,8 @@ __device__ __forceinline__ void decode_op(const Prog& P, int i, uint64_t base, i
     word = (s0 >= 0 && s0 < TB ? 1 << s0 : 0) | (s1 >= 0 && s1 < TB ? 1 << (s1 + 16) : 0);
     if (s1 >= 0 && s0 < 0) e[3] = e[2];
     const bool real = e[0].x != 0.f || e[1].x != 0.f || e[2].x != 0.f || e[3].x != 0.f;
-    if (s0 >= TB || (grad && real))
+    const bool unit = unit_modulus(e[0]) && unit_modulus(e[1]) && unit_modulus(e[2]) && unit_modulus(e[3]);
+    if (s0 >= TB || (grad && real) || (kReverse && !grad && !unit))
       cls = kGeneric;
     else
       cls = s1 >= TB ? (grad ? kGradElemReg : kElemReg) + (s1 - TB) : grad ? kGradElem : kElem;
@@ -128,6 +133,7 @@ __device__ __forceinline__ void decode_op(const Prog& P, int i, uint64_t base, i
     for (int q = 0; q < 4; ++q) {
       if (q >= k) break;
       e[q] = P.mats[mat + q];
+      if (kReverse && !unit_modulus(e[q])) cls = kGeneric;
       int lanes = 0, regs = 0;
       bool both = true;
 #pragma unroll
@@ -150,11 +156,11 @@ __device__ __forceinline__ void decode_op(const Prog& P, int i, uint64_t base, i
 }
 
 // Records of the pass's ops from `first` on (up to kStageOps), ended by kEnd.  Every thread takes part.
-template <int NT, class Prog>
+template <int NT, bool kReverse, class Prog>
 __device__ __forceinline__ void decode_program(const Prog& P, int first, uint64_t base, int* recs) {
   static_assert(kStageOps < NT, "one thread per op");
   const int left = P.op_count - first, n = left < kStageOps ? left : kStageOps;
-  if ((int)threadIdx.x < n) decode_op<__builtin_ctz(NT)>(P, first + threadIdx.x, base, recs + threadIdx.x * kRecWords);
+  if ((int)threadIdx.x < n) decode_op<__builtin_ctz(NT), kReverse>(P, first + threadIdx.x, base, recs + threadIdx.x * kRecWords);
   if ((int)threadIdx.x == n) recs[n * kRecWords] = kEnd;
   __syncthreads();
 }
@@ -400,14 +406,15 @@ __device__ __forceinline__ void adjoint_staged(float2 (&va)[PER], float2 (&vb)[P
 
 // pass_tile / adjoint_tile with the program decoded behind the tiles and the matrix stage, kStageOps ops
 // at a time.
-struct RunStaged {
+template <bool kReverse>
+struct RunDecoded {
   template <class Prog>
   static __device__ __forceinline__ int* records(const Prog& P, float2* mstage) {
     return reinterpret_cast<int*>(mstage + mstage_words(P.max_k));
   }
   template <int NT, class Prog>
   static __device__ __forceinline__ void begin(const Prog& P, uint64_t base, float2* mstage) {
-    decode_program<NT>(P, 0, base, records(P, mstage));
+    decode_program<NT, kReverse>(P, 0, base, records(P, mstage));
   }
   template <int PER, int NT, class Prog>
   static __device__ __forceinline__ void run(float2 (&v)[PER], float2* tile, float2* mstage, const Prog& P,
@@ -418,11 +425,12 @@ struct RunStaged {
       first += kStageOps;
       if (first >= P.op_count) return;
       __syncthreads();
-      decode_program<NT>(P, first, base, recs);
+      decode_program<NT, kReverse>(P, first, base, recs);
     }
   }
 };
-struct RunStagedAdjoint : RunStaged {
+using RunStaged = RunDecoded<false>;
+struct RunStagedAdjoint : RunDecoded<true> {
   template <int PER, int NT, int L, class Prog>
   static __device__ __forceinline__ void run(float2 (&va)[PER], float2 (&vb)[PER], float2* tA, float2* tB,
                                              float2* mstage, const Prog& P, uint64_t base, bool act,
@@ -433,7 +441,7 @@ struct RunStagedAdjoint : RunStaged {
       first += kStageOps;
       if (first >= P.op_count) return;
       __syncthreads();
-      decode_program<NT>(P, first, base, recs);
+      decode_program<NT, true>(P, first, base, recs);
     }
   }
 };

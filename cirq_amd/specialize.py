@@ -251,7 +251,8 @@ def _adj_mixing(op, nt: int, per: int) -> bool:
 
 
 def _in_diag_run(op) -> bool:
-    """Whether an op belongs to a run of diagonal ops: GRAD_DIAG, and DIAG or PAIRPHASE on both states."""
+    """Whether an op belongs to a run of diagonal ops: GRAD_DIAG, and DIAG or PAIRPHASE on both states (of unit
+    modulus: conj(phi) psi is then the same before and after)."""
     kind, sel = int(op["kind"]) & 0xFF, (int(op["kind"]) >> 8) & 3
     return kind == _lib.OP_GRAD_DIAG or (kind in (_OP_DIAG, _OP_PAIR) and sel == 0)
 
@@ -302,10 +303,25 @@ def _diag_run_source(index: int, ops, begin: int, end: int, tb: int) -> str:
     return "\n".join(out + ["  }"])
 
 
-def adjoint_pass_source(index: int, ps, ops: np.ndarray, n_bits: int) -> str:
+def _unit_modulus(packed) -> list:
+    """Per op, whether a DIAG or PAIRPHASE op's entries have modulus 1: those of fixed ops are read, those a gate's
+    parameters fill are a unitary's."""
+    filled = np.zeros(len(packed.mats_arr), dtype=bool)
+    for at, _, size in packed.param_entries:
+        filled[at : at + size] = True
+    out = []
+    for op in packed.ops_arr:
+        kind, k, at = int(op["kind"]) & 0xFF, int(op["k"]), int(op["mat"])
+        size = {_OP_DIAG: 1 << k, _OP_PAIR: k}.get(kind, 0)
+        entries = packed.mats_arr[at : at + size][~filled[at : at + size]]
+        out.append(bool(np.all(np.abs(np.abs(entries) ** 2 - 1) < 1e-6)))
+    return out
+
+
+def adjoint_pass_source(index: int, ps, ops: np.ndarray, n_bits: int, unit: list) -> str:
     """HIP source of one reverse-sweep pass as `extern "C" __global__ void k_aspec_<index>(float2*
     psi, float2* phi, TileProg, double* partial, int64_t stride)`, the same steps as adjoint.hpp
-    adjoint_tile for this pass's ops, on states of n_bits bits."""
+    adjoint_tile for this pass's ops, on states of n_bits bits.  unit: _unit_modulus of all ops."""
     L = int(ps["L"])
     nt, per = _shape(L)
     # The two tiles of up to 2^11 amplitudes leave room in LDS for four workgroups per CU, i.e. four waves per SIMD:
@@ -339,9 +355,9 @@ def adjoint_pass_source(index: int, ps, ops: np.ndarray, n_bits: int) -> str:
         op = ops[first + j]
         kind, sel = int(op["kind"]) & 0xFF, (int(op["kind"]) >> 8) & 3
         ref = f"kA{index}_{j}"
-        if _in_diag_run(op):
+        if _in_diag_run(op) and unit[first + j]:
             end = j
-            while end < count and _in_diag_run(ops[first + end]):
+            while end < count and _in_diag_run(ops[first + end]) and unit[first + end]:
                 end += 1
             body.append(_diag_run_source(index, ops[first : first + count], j, end, tb))
             j = end
@@ -456,7 +472,8 @@ def program_sources(packed, adjoint: bool = False) -> list[str]:
     head = f'#include "{CSRC / ("adjoint.hpp" if adjoint else "tile.hpp")}"\nusing namespace cqs;\n'
     ops = packed.ops_arr
     if adjoint:
-        kernels = [adjoint_pass_source(i, ps, ops, packed.n_bits) for i, ps in enumerate(packed.pass_arr)]
+        unit = _unit_modulus(packed)
+        kernels = [adjoint_pass_source(i, ps, ops, packed.n_bits, unit) for i, ps in enumerate(packed.pass_arr)]
     else:
         kernels = [pass_source(i, ps, ops) for i, ps in enumerate(packed.pass_arr)]
     per = 1 if adjoint else KERNELS_PER_FILE  # reverse-sweep kernels are several times larger

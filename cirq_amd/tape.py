@@ -962,12 +962,13 @@ class PackedProgram:
             for op in ps.ops:
                 if op.kind == "pair":
                     run_pairs.append(op)
-                elif op.kind in ("dense", "block", "grad_dense") or op.sel != 0:
+                elif (op.kind in ("dense", "block", "grad_dense") or op.sel != 0
+                      or op.kind == "grad_diag" and any(abs(abs(p.mat) ** 2 - 1) > 1e-6 for p in run_pairs)):
                     flush()
                     ops.append(op)
                 else:
                     # elementwise ops commute with the pending pair phases, and a diagonal gradient
-                    # does not see phases applied to both states
+                    # does not see phases (of modulus 1) applied to both states
                     ops.append(op)
             flush()
             out.append(Pass(ps.L, ps.lpos, ops))

@@ -43,8 +43,8 @@ extern "C" {
 #define CQS_OP_PAIRPHASE 3 /* product of phases on bit pairs (a CZ / CZPow layer)           */
 #define CQS_OP_SCALE 4     /* multiply every amplitude by one complex number (global phase) */
 #define CQS_OP_BLOCK 5     /* fused 2^k x 2^k block (k = 4 or 5) on MFMA, split-FP16 operands  */
-#define CQS_OP_GRAD_DENSE 6 /* adjoint only: partial of 2 Re<phi|dU|psi> for a dense dU (k <= 3) */
-#define CQS_OP_GRAD_DIAG 7  /* adjoint only: the same for a diagonal dU (DIAG bit encoding)     */
+#define CQS_OP_GRAD_DENSE 6 /* adjoint only: partial of 2 Re<phi|G|psi> for a dense G (k <= 3)  */
+#define CQS_OP_GRAD_DIAG 7  /* adjoint only: the same for a diagonal G (DIAG bit encoding)      */
 #define CQS_OP_PERMUTE 8    /* re-layout of the tile: tile bit b moves to tile bit aux[t[0] + b] */
 /* In adjoint programs bits 8-9 of `kind` select the tile an op acts on: 0 both, 1 psi, 2 phi. */
 
@@ -72,8 +72,11 @@ extern "C" {
  *              the same way; three products (hi*hi, lo*hi, hi*lo) accumulate in FP32.
  *   PERMUTE:   k = L; tile element j moves to the index whose bit aux[t[0] + b] is bit b of j.
  *              Later ops of the pass name tile bits in the new layout.  Forward passes only.
- *   slot:      parameter slot for gradient bookkeeping (-1 when unused); GRAD ops write their
- *              per-tile partial to grad_partial[slot * partial_stride + tile].
+ *   GRAD:      G is any matrix or diagonal (no local controls); the ops see both states as they are between the
+ *              ops before and after them.  For dU of a gate U, G = dU U^dagger before U is undone on both states.
+ *   slot:      parameter slot for gradient bookkeeping (-1 when unused); wave w of a tile's W waves writes its
+ *              share of a GRAD op to grad_partial[slot * partial_stride + tile * W + w], W = 4 for L <= 12,
+ *              2^(L - 10) above.
  */
 typedef struct cqs_op {
   int32_t kind;
@@ -95,8 +98,8 @@ typedef struct cqs_op {
  * reads and writes the state once.
  * Thread t of T holds tile elements t + e*T: the lowest log2(T) tile bits are thread bits, the
  * highest log2(2^L / T) are register bits.  DENSE ops with k <= 3 whose targets are all register
- * bits, given in ascending order, run in registers; other DENSE and BLOCK ops exchange the tile
- * through LDS.
+ * bits, given in ascending order, run in registers, and so do those with k = 1 on the six lowest tile bits
+ * (lanes of one wave); other DENSE and BLOCK ops exchange the tile through LDS.
  */
 typedef struct cqs_pass {
   int32_t L;
@@ -201,7 +204,8 @@ int cqs_adjoint_passes(void* psi, void* phi, int32_t n_bits, const cqs_pass* pas
 /* out[g] = sum over t < partial_stride of grad_partial[g * partial_stride + t], g < n_slots. */
 /*
  * cqs_adjoint_passes with reverse pass i run by kernels[i], a kernel compiled for that pass's op
- * sequence by cirq_amd/specialize.py (adjoint=True) against this library's csrc/adjoint.hpp:
+ * sequence by cirq_amd/specialize.py (adjoint=True) against this library's csrc/adjoint.hpp (diagonal ops on both
+ * states whose entries had modulus 1, or are filled by a gate's parameters, must keep it):
  * the host launch handle of a `__global__ void (float2* psi, float2* phi, TileProg, double*
  * partial, int64_t stride)`.  Arguments are checked as for cqs_adjoint_passes.  Same reference
  * (the reverse sweep of Jones & Gacon, arXiv:2009.02823; no Cirq counterpart).

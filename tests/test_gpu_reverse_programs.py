@@ -191,3 +191,18 @@ def test_programs_that_touch_one_state(gpu, sel, specialize):
            for t in ((9, 10), (0, 7), (3,), (7,))]
     for chosen in ([ops[0]], [ops[1]], ops):
         _check_program(gpu, rng, 12, 11, chosen, list(range(11)), specialize)
+
+
+@pytest.mark.parametrize("n,L,count,specialize", [(5, 5, 30, False), (9, 7, 64, False), (12, 11, 64, False), (13, 12, 40, False),
+                                                  (12, 11, 40, True)])
+def test_diagonal_ops_of_any_modulus(gpu, n, L, count, specialize):
+    """Gradients on both sides of diagonal ops that change conj(phi) psi (scales, diagonals, pairs on both states)."""
+    print(f"any modulus n={n} L={L} ops={count} specialize={specialize}", flush=True)
+    rng = np.random.RandomState(31 * n + L)
+    local = sorted(int(b) for b in rng.permutation(n)[:L])
+    ops = []
+    while len(ops) < count:
+        op = _random_op(rng, n, local, unit=False)
+        if "diag" in op.kind or op.kind in ("pair", "scale"):
+            ops.append(op)
+    _check_program(gpu, rng, n, L, ops, local, specialize, unit=False)
