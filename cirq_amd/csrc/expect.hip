@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <atomic>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include <string.h>
@@ -16,10 +17,10 @@ constexpr int kRedBlocks = 512;  // k_inner: fixed grid => deterministic reducti
 //
 // Term t needs sum_i s(i) conj(psi[i ^ x]) psi[i], s(i) = (-1)^popcount(i & z).  The indices i and
 // i ^ x give w s and conj(w) s (-1)^popcount(x & z), so the sum is 2 Re w or 2i Im w over half of the
-// indices: where x reaches above the chunk only the chunks with its highest bit clear do the work.
+// indices: where x reaches above the chunk, half of the chunks do the work.
 // A workgroup owns a slice of the state in chunks of 2^kChunkBits amplitudes and kPauliGroup terms: it holds
 // a chunk in registers and reads each term's partner chunk i ^ x (a permutation of one chunk, so reads
-// stay coalesced; terms with equal x share it), two amplitudes to a load.  The state is read about
+// stay coalesced; terms with equal x share it and its products), two amplitudes to a load.  The state is read about
 // 1 + kPauliGroup / 2 times per kPauliGroup terms, by workgroups that run side by side (the group is the
 // fastest grid index) and find it in cache.  What bounds it is the FP64 arithmetic and, for small
 // states, the launch: 200 4-local terms on 20 qubits take 160 us
@@ -28,13 +29,15 @@ constexpr int kRedBlocks = 512;  // k_inner: fixed grid => deterministic reducti
 constexpr int kPauliTerms = 96;   // arguments stay below 4 KB
 constexpr int kPauliGroup = 8;    // terms of one workgroup (FP64 accumulators in registers)
 constexpr int kChunkBits = 11;    // 256 threads x 4 pairs of amplitudes
-constexpr int kPauliSlices = 256; // fixed by n alone => deterministic reduction order
+constexpr int kPauliSlices = 512; // fixed by n alone => deterministic reduction order; two workgroups per CU for one group
+constexpr int kFewPauliTerms = 16;  // launches of so few take 0.6 KB of arguments each (3.4 KB: 3 us more for one term)
+template <int kMax>
 struct PauliBatch {
   int count;
-  int out_idx[kPauliTerms];
-  uint64_t x[kPauliTerms];
-  uint64_t z[kPauliTerms];
-  double cr[kPauliTerms], ci[kPauliTerms];
+  int out_idx[kMax];
+  uint64_t x[kMax];
+  uint64_t z[kMax];
+  double cr[kMax], ci[kMax];
 };
 
 // Amplitudes i and i + 1 (i even); `pairs`: the state starts on 16 bytes.
@@ -46,9 +49,9 @@ __device__ __forceinline__ float4 load_pair(const float2* amps, uint64_t i, int 
 
 // Writes out[out_idx] = c * sum when one slice covers the state, else the slice's share of every
 // term's sum to partials[(term * slices + slice) * 2 + {0,1}].  pre: as in k_expect_z (1 for density matrices).
-template <bool kDm>
-__global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ amps, int n, int slices,
-                                                     int pairs, float pre, PauliBatch tb, double* __restrict__ partials,
+template <bool kDm, int kMax>
+__global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ amps, int n, int slices, int pairs,
+                                                     float pre, PauliBatch<kMax> tb, double* __restrict__ partials,
                                                      double* __restrict__ out) {
   __shared__ double red[4][kPauliGroup][2];
   const uint64_t N = 1ull << n;
@@ -83,13 +86,24 @@ __global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ 
       }
     }
     float2 b[8];
+    double w[8];  // the products of the last term with another x mask, or another parity of Y
+    uint64_t px = ~0ull;
+    bool podd = false;
 #pragma unroll
     for (int t = 0; t < kPauliGroup; ++t) {
       if (t >= cnt) break;
       const uint64_t x = tb.x[t0 + t], z = tb.z[t0 + t];
-      // half of the chunks for an x that leaves the chunk (sums are doubled below)
-      if (!kDm && (x >> kChunkBits) != 0 && ((base >> (63 - __builtin_clzll(x))) & 1)) continue;
-      if (kDm || t == 0 || x != tb.x[t0 + t - 1]) {
+      // Half of the chunks for an x that leaves the chunk (sums are doubled below): of a chunk and its partner the one
+      // whose bit at the top of x equals the state's top bit, or, with that in x, the one where it is clear.  The
+      // top bit numbers a slice's chunks, so every slice does its share (X on bit 12 of 29: 3.1 ms; with
+      // the lower half of each pair, the chunks of half of the slices, 3.9 ms).
+      if (!kDm && (x >> kChunkBits) != 0) {
+        const int top = 63 - __builtin_clzll(x);
+        if (((base >> top) ^ (top < n - 1 ? base >> (n - 1) : 0)) & 1) continue;
+      }
+      const bool fresh = x != px, odd = __popcll(x & z) & 1;
+      px = x;
+      if (fresh) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const uint64_t i = base | ((uint64_t)e << 9) | (tid << 1);
@@ -109,7 +123,16 @@ __global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ 
           }
         }
       }
-      const bool odd = __popcll(x & z) & 1;
+      if constexpr (!kDm) {  // conj(b) a: its real part, or its imaginary part for an odd number of Y
+        if (fresh || odd != podd) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const double br = b[k].x * pre, bi = b[k].y * pre, xr = a[k].x * pre, xi = a[k].y * pre;
+            w[k] = odd ? fma(br, xi, -bi * xr) : fma(br, xr, bi * xi);
+          }
+        }
+        podd = odd;
+      }
       double sr = 0.0, si = 0.0;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -118,10 +141,8 @@ __global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ 
         if constexpr (kDm) {
           sr = fma(sg, (double)b[k].x, sr);
           si = fma(sg, (double)b[k].y, si);
-        } else {  // conj(b) a: its real part, or its imaginary part for an odd number of Y
-          const double br = b[k].x * pre, bi = b[k].y * pre, xr = a[k].x * pre, xi = a[k].y * pre;
-          const double w = odd ? fma(br, xi, -bi * xr) : fma(br, xr, bi * xi);
-          sr = fma(sg, w, sr);
+        } else {
+          sr = fma(sg, w[k], sr);
         }
       }
       const bool neg = (((tneg >> t) & 1) ^ (__popcll(base & z) & 1)) != 0;
@@ -161,7 +182,8 @@ __global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ 
 }
 
 // One wave per term sums its slices in a fixed order.
-__global__ __launch_bounds__(64) void k_pauli_final(const double* __restrict__ partials, int slices, PauliBatch tb,
+template <int kMax>
+__global__ __launch_bounds__(64) void k_pauli_final(const double* __restrict__ partials, int slices, PauliBatch<kMax> tb,
                                                     double* __restrict__ out) {
   const int t = blockIdx.x;
   double sr = 0.0, si = 0.0;
@@ -424,34 +446,39 @@ static int expect_batches(const void* amps, int32_t n_qubits, int32_t is_dm, int
       hipLaunchKernelGGL(k_expect_z_final, dim3(zf.count), dim3(64), 0, s, (const double*)partials, zf, out);
       continue;
     }
-    PauliBatch tb;
-    memset(&tb, 0, sizeof(tb));
-    for (; i < n_terms && tb.count < kPauliTerms && !z_only(i); ++i) {
-      const int t = term(i);
-      tb.x[tb.count] = xmask[t];
-      tb.z[tb.count] = zmask[t];
-      tb.out_idx[tb.count] = t;
-      tb.cr[tb.count] = coef[2 * t];
-      tb.ci[tb.count] = coef[2 * t + 1];
-      ++tb.count;
-    }
-    const int pairs = (reinterpret_cast<uintptr_t>(amps) & 15) == 0;
-    const dim3 grid((tb.count + kPauliGroup - 1) / kPauliGroup * slices);
-    if (is_dm)
-      hipLaunchKernelGGL(k_pauli_terms<true>, grid, dim3(256), 0, s, (const float2*)amps, (int)n_qubits, slices,
-                         pairs, pre, tb, partials, out);
+    const int first = i;
+    while (i < n_terms && i - first < kPauliTerms && !z_only(i)) ++i;
+    auto launch = [&](auto max) {
+      constexpr int kMax = decltype(max)::value;
+      PauliBatch<kMax> tb;
+      memset(&tb, 0, sizeof(tb));
+      for (; tb.count < i - first; ++tb.count) {
+        const int t = term(first + tb.count);
+        tb.x[tb.count] = xmask[t];
+        tb.z[tb.count] = zmask[t];
+        tb.out_idx[tb.count] = t;
+        tb.cr[tb.count] = coef[2 * t];
+        tb.ci[tb.count] = coef[2 * t + 1];
+      }
+      const int pairs = (reinterpret_cast<uintptr_t>(amps) & 15) == 0;
+      const dim3 grid((tb.count + kPauliGroup - 1) / kPauliGroup * slices);
+      const auto kernel = is_dm ? &k_pauli_terms<true, kMax> : &k_pauli_terms<false, kMax>;
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, (const float2*)amps, (int)n_qubits, slices, pairs, pre, tb,
+                         partials, out);
+      if (slices > 1)
+        hipLaunchKernelGGL(k_pauli_final<kMax>, dim3(tb.count), dim3(64), 0, s, (const double*)partials, slices, tb, out);
+    };
+    if (i - first <= kFewPauliTerms)
+      launch(std::integral_constant<int, kFewPauliTerms>());
     else
-      hipLaunchKernelGGL(k_pauli_terms<false>, grid, dim3(256), 0, s, (const float2*)amps, (int)n_qubits, slices,
-                         pairs, pre, tb, partials, out);
-    if (slices > 1)
-      hipLaunchKernelGGL(k_pauli_final, dim3(tb.count), dim3(64), 0, s, (const double*)partials, slices, tb, out);
+      launch(std::integral_constant<int, kPauliTerms>());
   }
   CQS_HIP(hipGetLastError());
   return CQS_OK;
 }
 
 // Static scratch for cqs_expect_paulis_noalloc: one launch's partial sums, the largest any batch
-// writes (2048 blocks x 64 Z terms, or 256 slices x 96 terms x 2 doubles): 1 MiB per GPU, held
+// writes (2048 blocks x 64 Z terms, or 512 slices x 96 terms x 2 doubles): 1 MiB per GPU, held
 // until the process ends.  In host code `scratch` is only a handle for hipGetSymbolAddress; the
 // kernels get the device address that call returns, kept per device.
 static __device__ __align__(256) double scratch[kZBatch * kZBlocks];

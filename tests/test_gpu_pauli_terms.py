@@ -82,3 +82,24 @@ def test_norm_of_the_scaled_state_without_writing_it(gpu, n):
         t = st.clone()
         engine.scale(t, n, s)
         assert engine.norm2(st, n, ws, scale=s) == engine.norm2(t, n, ws)
+
+
+@pytest.mark.parametrize("n,offset", [(21, 0), (22, 1)])
+def test_terms_of_states_with_several_chunks_per_slice(gpu, n, offset):
+    """Masks whose top bit numbers a slice, a slice's chunks, the state's halves; equal masks with either parity of Y in a
+    row; 16 terms (the small argument block) and more."""
+    rng = np.random.RandomState(n)
+    psi = (rng.randn(2**n) + 1j * rng.randn(2**n)).astype(np.complex64)
+    psi /= np.linalg.norm(psi)
+    buf = torch.empty(2**n + offset, dtype=torch.complex64, device=gpu)
+    st = buf[offset:]
+    st.copy_(torch.from_numpy(psi))
+    xs = [1 << 12, 1 << 12, (1 << 12) | 3, 1 << 19, (1 << 20) | 1, 1 << (n - 1), (1 << (n - 1)) | (1 << 11), (1 << n) - 1, 5, 5, 5, 5]
+    zs = [0, 1 << 12, 1 << 20, (1 << 19) | 1, 1 << 20, 1 << (n - 1), 7, (1 << n) - 1, 0, 1, 4, 5]
+    xm, zm = np.array(xs, dtype=np.uint64), np.array(zs, dtype=np.uint64)
+    p, idx = psi.astype(np.complex128), np.arange(2**n, dtype=np.uint64)
+    want = np.array([np.sum(np.conj(p[(idx ^ x).astype(np.int64)]) * _signs(idx, z) * p) for x, z in zip(xm, zm)])
+    for count in (1, 12, 16, 17, 30):
+        pick = np.arange(count) % len(xs) if count > 1 else np.array([0])
+        got = _run(st, n, False, xm[pick], zm[pick], np.tile([1.0, 0.0], count))
+        assert np.abs(got - want[pick]).max() < 1e-13 * n  # as above
