@@ -1078,7 +1078,16 @@ __global__ __launch_bounds__(256) void k_perm_probs(const float2* __restrict__ a
 // doubling of S) it adds that block's elements one by one.  S after each of up to 256 segments is
 // kept, so the draw rescans one segment.  Bound by the latency of one block's chain (load, divide, tree):
 // 512 rows of 2^16 take 0.25 ms against 19.7 ms with a thread per row, 1,024 of 2^10 42 against 302 us.
-constexpr int kRowThreadBits = 6;  // 32,768 rows of 2^6: 61 us with a thread per row, 160 with a wave (1,024: 24, 17)
+//
+// A thread per row where rows are short and many.  Thread / wave per row in us: 2^6 entries, 1,024 rows 24 / 17,
+// 32,768 rows 61 / 160 (kernel alone); with sums and copies 2^7, 1,024 rows 102 / 83, 8,192 rows 113 / 129,
+// 32,768 rows 171 / 291; 2^8, 8,192 rows 149 / 158, 32,768 rows 216 / 375; 2^9, 8,192 rows 229 / 167, 32,768 rows
+// 303 / 401; 2^10, 32,768 rows 468 / 441.  A wave's time grows with the rows once they fill the chip, a thread's with
+// the row's length: the line is at 32 rows per entry, up to 2^9 entries.
+constexpr int kRowThreadBits = 6, kManyRowsBits = 9, kRowsPerEntry = 32;
+inline bool thread_per_row(int m, int64_t rows) {
+  return m <= kRowThreadBits || (m <= kManyRowsBits && rows >= ((int64_t)kRowsPerEntry << m));
+}
 __global__ __launch_bounds__(64) void k_draw_short_rows(const float* __restrict__ probs, int m, int n_rows,
                                                         const float* __restrict__ bsum,
                                                         const double* __restrict__ uni,
@@ -1489,7 +1498,7 @@ int cqs_draw_rows(const float* probs, int32_t m, int32_t n_rows, const double* u
   const Loader ld = make_loader(nullptr, probs, 0, 0);
   float* bsum = (float*)workspace;
   hipLaunchKernelGGL(k_sum_buffers, dim3((unsigned)nbuf), dim3(256), 0, s, ld, buflen, bsum);
-  if (m <= kRowThreadBits)
+  if (thread_per_row(m, n_rows))
     hipLaunchKernelGGL(k_draw_short_rows, dim3((unsigned)((n_rows + 63) / 64)), dim3(64), 0, s, probs, (int)m,
                        (int)n_rows, (const float*)bsum, uniforms, out_index, out_p);
   else

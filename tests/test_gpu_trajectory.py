@@ -430,3 +430,26 @@ def test_draw_rows_at_ties_and_binade_edges(gpu, m, shift):
         cdf /= cdf[-1]
         want = int(cdf.searchsorted(u[r], side="right"))  # RandomState.choice for the uniform u[r]
         assert idx[r] == want and p[r] == pr[want], (r, idx[r], want)
+
+
+@pytest.mark.parametrize("m,rows", [(7, 4095), (7, 4096), (8, 9000), (9, 700)])
+def test_draw_rows_short_and_many(gpu, m, rows):
+    """cqs_draw_rows on both sides of the line between a thread and a wave per row, against NumPy's cdf."""
+    _log(f"draw rows m={m} rows={rows}")
+    import torch
+
+    from cirq_amd import engine
+
+    rng = np.random.RandomState(rows)
+    q = rng.exponential(size=(rows, 2**m)).astype(np.float32)
+    q[::3] = np.ldexp(np.float32(1), -rng.randint(1, 60, q[::3].shape))  # powers of two: ties in the running sum
+    q[1::7, : 2 ** (m - 1)] = 0
+    p = q / q.sum(axis=1, keepdims=True)
+    cdf = p.astype(np.float64).cumsum(axis=1)
+    cdf /= cdf[:, -1:]
+    at = rng.randint(0, 2**m, rows)
+    u = np.where(rng.rand(rows) < 0.5, rng.random_sample(rows), cdf[np.arange(rows), at])
+    u = np.minimum(u, np.nextafter(1.0, 0))
+    idx, pr = engine.draw_rows(torch.from_numpy(q).cuda(), u, engine.Workspace(torch.device("cuda")))
+    want = np.sum(cdf <= u[:, None], axis=1)  # searchsorted, right
+    assert np.array_equal(idx, want) and np.array_equal(pr, p[np.arange(rows), want])
