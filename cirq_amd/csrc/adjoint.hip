@@ -4,10 +4,12 @@
 
 namespace cqs {
 
-template <int L>
-__global__ __launch_bounds__(TileShape<L>::NT) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_adjoint_pass(float2* __restrict__ psi, float2* __restrict__ phi,
-                                                                 TileProg P, double* __restrict__ partial,
-                                                                 int64_t stride) {
+// kWaves: the most waves per SIMD that registers are planned for.  Up to 11-bit tiles three give the MFMA blocks registers to
+// load ahead, where each CU has at most two workgroups anyway (20 qubits, passes of two-bit gates and blocks: 170 us a
+// sweep against 187); four hide more on many tiles (22 qubits 398 against 423 us, 24 qubits 1.30 against 1.45 ms).
+template <int L, int kWaves = (L <= 11 ? 3 : 8)>
+__global__ __launch_bounds__(TileShape<L>::NT) __attribute__((amdgpu_waves_per_eu(2, kWaves))) void k_adjoint_pass(
+    float2* __restrict__ psi, float2* __restrict__ phi, TileProg P, double* __restrict__ partial, int64_t stride) {
   extern __shared__ float2 lds[];
   const uint64_t base = deposit_bounded<31>((uint64_t)blockIdx.x, P.opos, P.nouter);
   adjoint_tile<L>(psi, phi, P, P.lpos, base, partial, stride, blockIdx.x, lds);
@@ -15,9 +17,9 @@ __global__ __launch_bounds__(TileShape<L>::NT) __attribute__((amdgpu_waves_per_e
 
 typedef void (*AdjKernel)(float2*, float2*, TileProg, double*, int64_t);
 static const AdjKernel kAdjKernels[15] = {
-    k_adjoint_pass<0>, k_adjoint_pass<1>, k_adjoint_pass<2>, k_adjoint_pass<3>,  k_adjoint_pass<4>,
-    k_adjoint_pass<5>, nullptr,           nullptr,           nullptr,            nullptr,
-    nullptr,           nullptr,           k_adjoint_pass<12>, k_adjoint_pass<13>, k_adjoint_pass<14>};  // 6-11: kAdjStaged
+    k_adjoint_pass<0>,  k_adjoint_pass<1>,  k_adjoint_pass<2>,  k_adjoint_pass<3>,  k_adjoint_pass<4>,
+    k_adjoint_pass<5>,  k_adjoint_pass<6>,  k_adjoint_pass<7>,  k_adjoint_pass<8>,  k_adjoint_pass<9>,
+    k_adjoint_pass<10>, k_adjoint_pass<11>, k_adjoint_pass<12>, k_adjoint_pass<13>, k_adjoint_pass<14>};
 
 // out[g] = sum_t partial[g * ntiles + t]  (fixed order)
 __global__ __launch_bounds__(64) void k_grad_reduce(const double* __restrict__ partial, int64_t ntiles,
@@ -58,10 +60,12 @@ static int adjoint_passes(void* psi, void* phi, int32_t n_bits, const cqs_pass* 
                 (long long)entries);
     const int mk = ps.max_k;
     const size_t stage = mk >= 3 ? (size_t(1) << (2 * mk)) : 0;
-    const bool staged = kernels == nullptr && staged_adjoint_width(ps.L);
+    const bool staged = kernels == nullptr && staged_adjoint_pass(P);
     const size_t shmem =
         (2 * (size_t)tile_words(ps.L) + stage) * sizeof(float2) + (staged ? kStagedBytes : 0);
-    const AdjKernel kernel = staged ? kAdjStaged[ps.L] : kAdjKernels[ps.L];
+    const AdjKernel kernel = staged                         ? kAdjStaged[ps.L]
+                             : ps.L == 11 && P.nouter > 9 ? (AdjKernel)k_adjoint_pass<11, 8>
+                                                          : kAdjKernels[ps.L];
     CQS_REQUIRE(shmem <= 160 * 1024 - 1024, "adjoint pass needs %zu bytes of LDS", shmem);
     if (shmem > 64 * 1024)
       CQS_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));

@@ -8,7 +8,7 @@
 // outer bits of diagonals and phases), small matrices lie in the record, and a class number selects
 // the code.  Ops without a class of their own run through the functions of tile.hpp and adjoint.hpp.
 // A one-bit gate takes 0.32 us instead of 0.74 on 10 qubits, a diagonal 0.37 instead of 0.68; the gradient of
-// a 20-qubit ansatz 1.8 ms instead of 2.2, of a 13-qubit one (4 rows) 1.95 instead of 2.5.
+// a 20-qubit ansatz 1.92 ms instead of 2.24, of a 13-qubit one (4 rows) 2.04 instead of 2.50.
 #pragma once
 
 #include "adjoint.hpp"
@@ -456,14 +456,21 @@ constexpr int kStagedMinL = 6, kStagedMaxL = 12;
 constexpr int kStagedAdjMaxL = 11;  // two states of 16 elements per thread spill 400 registers here
 constexpr bool staged_adjoint_width(int L) { return L >= kStagedMinL && L <= kStagedAdjMaxL; }
 constexpr bool staged_width(int L) { return L >= kStagedMinL && L <= kStagedMaxL; }
-// Forward passes that are decoded first: few tiles, or many ops.  Where MFMA blocks do the work of a large
-// state (a grid circuit's pass has 5-10 ops), the loop over scalar reads is the faster: 28 qubits, 16
-// cycles, 12-bit tiles 17.6 against 18.3 ms, 14-qubit density matrix 7.8 against 8.4; ansatz passes of 60-120 ops
-// at 28 qubits take 11.8 ms decoded against 13.9, at 2^10 tiles 0.29 against 0.30.  Reverse passes are always decoded
-// (24 qubits: 4.3 against 8.4 ms).
-constexpr int kStagedOuterBits = 10, kStagedManyOps = 32;
-inline bool staged_pass(const TileProg& P) {
-  return staged_width(P.L) && (P.nouter <= kStagedOuterBits || P.op_count >= kStagedManyOps);
+// Passes that are decoded first: those of many ops.  Decoding costs a start (0.3-1 us on few tiles, a tenth of a
+// pass of 2-4 ops) and 0.1-0.2 us more for each op without a class of its own, and saves 0.2-0.4 us for each op with one.  The
+// host does not see the kinds (ops lie on the device), but programs of one-bit gates have long passes, and those whose gates
+// fuse into two-bit matrices and MFMA blocks short ones: grid circuits and noisy density matrices 1-14 ops.  Scalar /
+// decoded in us: 16 one-bit and diagonal ops 14.0 / 10.2 on 10 qubits, 23.0 / 18.1 on 20, 31.3 / 31.0 on 22; 8 blocks and
+// phases 10.9 / 11.4, 19.7 / 20.4, 30.2 / 33.2; 16 of them 19.1 / 19.0, 34.2 / 34.5, 52.5 / 56.3.  On more tiles the waves hide
+// more of the scalar decoding: 16 gates 56 / 54 on 23 qubits, 368 / 357 on 26, 32 gates 100 / 91 and 689 / 627.
+// The same in reverse passes: 8 gates and gradients 12.6 / 9.2 on 10 qubits, 18.0 / 15.3 on 20, 130 / 132 on 24, 16 of
+// them 22.1 / 13.8, 29.2 / 22.2, 226 / 201; 4 blocks 11.7 / 13.0, 17.4 / 19.5, 145 / 187, 16 blocks, gradients and phases
+// 29.5 / 25.8, 38.8 / 38.5, 335 / 392, 32 of them 54.4 / 44.9, 68.5 / 66.2, 617 / 702.
+constexpr int kStagedOuterBits = 10, kStagedOps = 16, kStagedManyOps = 32;
+inline bool staged_ops(const TileProg& P) {
+  return P.op_count >= (P.nouter <= kStagedOuterBits ? kStagedOps : kStagedManyOps);
 }
+inline bool staged_pass(const TileProg& P) { return staged_width(P.L) && staged_ops(P); }
+inline bool staged_adjoint_pass(const TileProg& P) { return staged_adjoint_width(P.L) && staged_ops(P); }
 
 }  // namespace cqs

