@@ -52,18 +52,15 @@ def _dagger(kind: str, x):
     return np.conj(x)
 
 
-def _inverse(op: LOp, sel: int) -> LOp:
-    """U^dagger on the states `sel` selects.  One-state inverses ask for their controls as local
-    bits too, so that the two of a pair share a pass.  (Split across passes, another op's gradient
-    could run while only one of the two states had this inverse applied.)"""
+def _inverse(op: LOp) -> LOp:
+    """U^dagger on both states."""
     if op.kind == "scale" and abs(abs(complex(op.mat)) - 1) > 1e-9:
         raise ValueError("adjoint gradients need a unitary circuit (non-unit scale factor)")
     ref = op.pref
     if ref is not None:
         base, kind = ref.transform, op.kind
         ref = ParamRef(ref.gate, lambda b, base=base, kind=kind: _dagger(kind, base(b)), ref.exprs, ref.slot)
-    need = tuple(b for b, _ in op.controls) if sel != _lib.SEL_BOTH else ()
-    return LOp(op.kind, op.targets, _dagger(op.kind, op.mat), op.controls, ref, sel, need=need)
+    return LOp(op.kind, op.targets, _dagger(op.kind, op.mat), op.controls, ref)
 
 
 def _constant_generator(gate):
@@ -191,14 +188,14 @@ class AdjointProgram:
         self.grad_slots: list[tuple[ParamRef, int]] = []  # slot -> (forward op's ref, parameter index)
         for op in reversed(low.ops):
             if op.fixed:
-                rev.append(_inverse(op, _lib.SEL_BOTH))
+                rev.append(_inverse(op))
                 continue
             for k, e in enumerate(op.pref.exprs):
                 if is_parameterized(e):
                     slot = len(self.grad_slots)
                     self.grad_slots.append((op.pref, k))
                     rev.append(_grad_op(op, k, slot))
-            rev.append(_inverse(op, _lib.SEL_BOTH))
+            rev.append(_inverse(op))
         rev = fuse_single_bit(rev)
         passes = schedule(rev, n, La, coalesce_bits)
         if mfma_blocks:

@@ -71,8 +71,9 @@ def _inverse_norm(op: LOp) -> float:
 
 
 def _undo_pair(op: LOp) -> list[LOp]:
-    """S^-1 on rho and S^dagger on lambda for an invertible channel or scale op (same bits, so
-    the scheduler keeps them in one pass)."""
+    """S^-1 on rho and S^dagger on lambda for an invertible channel or scale op: the only ops that undo
+    something on one state at a time.  They act on the same bits and follow each other, so the scheduler takes or
+    defers both and no gradient op runs between them (there the two states would not belong together)."""
     if op.kind == "scale":
         c = complex(op.mat)
         return [LOp("scale", (), np.complex128(1 / c), (), None, _lib.SEL_PSI),
@@ -172,14 +173,14 @@ class DMAdjointProgram:
                     rev += _undo_pair(op)
                     continue
                 if op.fixed:
-                    rev.append(_inverse(op, _lib.SEL_BOTH))
+                    rev.append(_inverse(op))
                     continue
                 for k, e in enumerate(op.pref.exprs):
                     if is_parameterized(e):
                         slot = len(self.grad_slots)
                         self.grad_slots.append((op.pref, k))
                         rev.append(_grad_op(op, k, slot))
-                rev.append(_inverse(op, _lib.SEL_BOTH))
+                rev.append(_inverse(op))
             if chan is not None:
                 rev.append(_adjoint_of_nonunitary(chan))
             a = len(rev_passes)

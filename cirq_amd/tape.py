@@ -29,19 +29,16 @@ OUTER = 64  # DIAG / PAIRPHASE bit encoding: tile-local index, or OUTER + global
 
 @dataclasses.dataclass(frozen=True)
 class Generator:
-    """In ParamRef.deriv: evaluate dM/d(parameter k) M^dagger of the gate's matrix M."""
+    """dM/d(parameter k) M^dagger of a gate's matrix M."""
 
     k: int
 
 
-def gate_matrices(gate, vals: tuple, deriv) -> np.ndarray:
-    """(B, d, d): the gate's matrices at the parameter values (deriv None), their derivatives in
-    parameter `deriv`, or the products of those with the inverse matrices (a Generator)."""
+def gate_matrices(gate, vals: tuple, deriv: Generator | None) -> np.ndarray:
+    """(B, d, d): the gate's matrices at the parameter values, or the generators of one parameter there."""
     if deriv is None:
         return np.asarray(gate._matrix_batch(vals))
-    if isinstance(deriv, Generator):
-        return gate._dmatrix_batch(vals, deriv.k) @ np.conj(np.swapaxes(gate._matrix_batch(vals), -1, -2))
-    return np.asarray(gate._dmatrix_batch(vals, deriv))
+    return gate._dmatrix_batch(vals, deriv.k) @ np.conj(np.swapaxes(gate._matrix_batch(vals), -1, -2))
 
 
 @dataclasses.dataclass
@@ -56,7 +53,7 @@ class ParamRef:
     transform: Callable
     exprs: tuple
     slot: int = -1
-    deriv: int | Generator | None = None  # evaluate a derivative or generator instead of the matrix
+    deriv: Generator | None = None  # evaluate a parameter's generator instead of the matrix
 
 
 @dataclasses.dataclass
@@ -70,7 +67,6 @@ class LOp:
     slot: int = -1  # adjoint GRAD ops: gradient slot
     vbits: tuple = ()  # fused dense / block ops: outer bits selecting one of 2^len matrices (mat[v])
     fence: bool = False  # scheduling barrier: runs after every earlier op, before every later one
-    need: tuple = ()  # bits that must be local in the op's pass besides its targets
 
     @property
     def bits(self) -> frozenset:
@@ -337,12 +333,11 @@ class Lowering:
         self.ops.append(LOp("dense", cols + rows, sop))
 
 
-def _sub_ref(ref: ParamRef | None, transform, deriv: int | None = None):
+def _sub_ref(ref: ParamRef | None, transform):
     if ref is None:
         return None
     base = ref.transform
-    return ParamRef(ref.gate, lambda b, base=base: transform(base(b)), ref.exprs, ref.slot,
-                    ref.deriv if deriv is None else deriv)
+    return ParamRef(ref.gate, lambda b, base=base: transform(base(b)), ref.exprs, ref.slot, ref.deriv)
 
 
 # --------------------------------------------------------------------------------------------
@@ -723,7 +718,7 @@ def schedule(ops: list[LOp], n_bits: int, L: int, coalesce: int) -> list[Pass]:
                 blocked |= bits
                 continue
             if op.kind in ("dense", "grad_dense"):
-                need = (set(op.targets) | set(op.need)) - S
+                need = set(op.targets) - S
                 if len(S) + len(need) <= L:
                     S |= need
                     take.append(op)
@@ -1473,7 +1468,7 @@ class ParamPlan:
 
     @staticmethod
     def _group_matrices(rep, exprs, symvals):
-        """(G * B, d, d) matrices (or derivatives) of the group's gates, gate-major."""
+        """(G * B, d, d) matrices (or generators) of the group's gates, gate-major."""
         vals = tuple(e(symvals).reshape(-1) for e in exprs)
         return gate_matrices(rep.gate, vals, rep.deriv)
 

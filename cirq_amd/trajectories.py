@@ -34,12 +34,11 @@ MAX_KRAUS = 16
 
 
 # ---------------------------------------------------------------- NumPy's draws, vectorised
-def choice_rows(p: np.ndarray, u: np.ndarray) -> np.ndarray:
-    """Row r: RandomState.choice(len(p[r]), p=p[r]) given that its uniform is u[r]: the cumulative
-    sum in float64 normalised by its last entry, then searchsorted(..., 'right')."""
-    cdf = np.cumsum(np.asarray(p, dtype=np.float64), axis=-1)
-    cdf = cdf / cdf[..., -1:]
-    return np.sum(cdf <= np.asarray(u, dtype=np.float64)[:, None], axis=-1).astype(np.int64)
+def choice_cdf(p: np.ndarray) -> np.ndarray:
+    """What RandomState.choice(len(p), p=p) searches for its uniform (side 'right'): the cumulative sum in float64
+    normalised by its last entry."""
+    cdf = np.cumsum(np.asarray(p, dtype=np.float64))
+    return cdf / cdf[-1]
 
 
 def kraus_draws(weights: np.ndarray, u: np.ndarray) -> tuple[np.ndarray, np.ndarray]:
@@ -250,9 +249,18 @@ class TrajectoryBatch:
                     groups.setdefault(key, (probs, self._identity[j], []))[2].append(j)
             self._groups = []
             for probs, identity, js in groups.values():
-                cdf = np.cumsum(probs)
-                self._groups.append((cdf / cdf[-1], identity, np.array(js)))
+                self._groups.append((choice_cdf(probs), identity, np.array(js)))
         return self._groups
+
+    def _mixture_table(self, u: np.ndarray) -> np.ndarray:
+        """Row j: every copy's matrix of stochastic op j for the uniforms u (copies, ops) if that is a mixture, -1 (also
+        for other ops) where it is the identity, which the kernels do not touch."""
+        R, D = u.shape
+        table = np.full((max(D, 1), R), -1, dtype=np.int32)
+        for cdf, identity, js in self._mixture_groups():
+            drawn = cdf.searchsorted(u[:, js].T, side="right")
+            table[js] = np.where(identity[drawn], -1, drawn)
+        return table
 
     def _run_batch(self, state0: torch.Tensor, resolver, R: int, u: np.ndarray) -> list:
         copy_bits = R.bit_length() - 1
@@ -261,11 +269,7 @@ class TrajectoryBatch:
         # a mixture's draw does not depend on the state: every copy's choice for every mixture is
         # known now and goes to the device in one copy (row j: stochastic op j)
         D = u.shape[1]
-        table = np.full((max(D, 1), R), -1, dtype=np.int32)
-        for cdf, identity, js in self._mixture_groups():
-            drawn = cdf.searchsorted(u[:, js].T, side="right")
-            # a drawn identity leaves the copy alone: -1, which the kernels do not touch
-            table[js] = np.where(identity[drawn], -1, drawn)
+        table = self._mixture_table(u)
         table_dev = engine._dev_array(table, self.device)
         ones = torch.ones(R, dtype=torch.float32, device=self.device)
         u_dev = engine._dev_array(np.ascontiguousarray(u.T), self.device) if D else None  # row j: op j
@@ -344,4 +348,4 @@ class TrajectoryBatch:
         engine.apply_select_batch_dev(states, self.n_bits, R, targets, m_dev, n_mats, sel, scl)
 
 
-__all__ = ["TrajectoryBatch", "choice_rows", "kraus_draws"]
+__all__ = ["TrajectoryBatch", "choice_cdf", "kraus_draws"]

@@ -7,11 +7,11 @@ Kraus walk of cirq-core/cirq/sim/state_vector_simulation_state.py:224-250) would
 import numpy as np
 import pytest
 
-from cirq_amd.trajectories import TrajectoryBatch, choice_rows, kraus_draws
+from cirq_amd.trajectories import TrajectoryBatch, choice_cdf, kraus_draws
 
 
 @pytest.mark.parametrize("seed", range(5))
-def test_choice_rows_matches_randomstate_choice(seed):
+def test_choice_cdf_matches_randomstate_choice(seed):
     rng = np.random.RandomState(100 + seed)
     R, K = 300, int(rng.randint(1, 17))
     p = rng.exponential(size=(R, K))
@@ -21,9 +21,36 @@ def test_choice_rows_matches_randomstate_choice(seed):
     a = np.random.RandomState(seed)
     want = np.array([a.choice(K, p=row) for row in p])
     b = np.random.RandomState(seed)
-    got = choice_rows(p, b.random_sample(R))
+    got = [choice_cdf(row).searchsorted(u, side="right") for row, u in zip(p, b.random_sample(R))]
     assert np.array_equal(got, want)
     assert a.random_sample() == b.random_sample()  # the same number of draws was consumed
+
+
+def test_mixture_table_holds_the_draws_of_every_mixture():
+    """The table that a batch's mixtures run by: RandomState.choice's outcome per copy and op, -1 for identities and for ops
+    that are no mixtures, whichever ops share probabilities."""
+    import torch
+
+    import cirq_amd as cirq
+
+    q = cirq.LineQubit.range(3)
+    ops = [cirq.depolarize(0.3)(q[0]), cirq.amplitude_damp(0.2)(q[1]), cirq.bit_flip(0.4)(q[1]), cirq.depolarize(0.3)(q[2]),
+           cirq.phase_flip(0.25)(q[0]), cirq.measure(q[0], key="m"), cirq.depolarize(0.9, 2)(q[0], q[2])]
+    batch = TrajectoryBatch(q, [("op", op) for op in ops], False, torch.device("cpu"), None, True, True, None)
+    batch._steps()
+    u = np.random.RandomState(3).random_sample((400, len(ops)))
+    table = batch._mixture_table(u)
+    assert table.shape == (len(ops), 400)
+    for j, op in enumerate(ops):
+        mix = None if j in (1, 5) else op.gate._mixture_()
+        for r in range(0, 400, 7):
+            if mix is None:
+                assert table[j, r] == -1
+                continue
+            p, mats = zip(*mix)
+            cdf = np.cumsum(p)
+            k = int((cdf / cdf[-1]).searchsorted(u[r, j], side="right"))
+            assert table[j, r] == (-1 if np.allclose(mats[k], np.eye(len(mats[k]))) else k)
 
 
 def _kraus_walk(weights_row, p):
