@@ -11,6 +11,7 @@ import cirq_amd as cirq
 from cirq_amd import engine
 from cirq_amd.adjoint import AdjointGradient
 from cirq_amd.tape import LOp, compile_ops
+from tests.test_adjoint_host import _oracle_grad
 
 pytestmark = pytest.mark.gpu
 
@@ -51,8 +52,8 @@ def test_one_bit_ops_on_every_tile_bit(gpu, n, L, specialize):
 
 @pytest.mark.parametrize("n,specialize", [(1, False), (2, False), (5, False), (7, False), (8, False), (9, True), (11, False), (12, True)])
 def test_gradients_on_every_bit(gpu, n, specialize):
-    """Rotations about X, Y, Z, controlled and diagonal pairs on every qubit: the adjoint sweep against
-    the two-term shift rule (controlled rotations, which have no such rule, stay fixed there)."""
+    """Rotations about X, Y, Z and diagonal pairs on every qubit, beside fixed CZ and CNOT: the adjoint sweep against
+    the two-term shift rule (controlled rotations, which have no such rule, are below)."""
     print(f"gradients n={n}", flush=True)
     rng = np.random.RandomState(n)
     qs = cirq.LineQubit.range(n)
@@ -79,3 +80,39 @@ def test_gradients_on_every_bit(gpu, n, specialize):
     v2, g2 = ag.parameter_shift(x)
     # complex64 states of about 10 n gates; H's coefficients sum to about 2 n
     assert abs(v - v2) < 1e-5 * n and np.abs(g - g2).max() < 1e-5 * n
+
+
+@pytest.mark.parametrize("n,L,specialize", [(3, None, False), (5, None, False), (7, 6, False), (9, 8, False), (9, 8, True), (9, 9, False)])
+def test_gradients_of_controlled_rotations(gpu, n, L, specialize):
+    """Generators with controls folded in (two- and three-bit gradient ops) and diagonal ones, on thread, register and
+    outer bits, against central differences of complex128 simulations."""
+    print(f"controlled gradients n={n} L={L}", flush=True)
+    rng = np.random.RandomState(n)
+    qs = cirq.LineQubit.range(n)
+    c, syms = cirq.Circuit([cirq.H(q) for q in qs]), []
+
+    def sym():
+        syms.append(sympy.Symbol(f"p{len(syms):03d}"))
+        return syms[-1]
+
+    for i in range(n):
+        a, b, d = (qs[int(x)] for x in rng.permutation(n)[:3])
+        c.append([cirq.ControlledGate(cirq.ry(sym())).on(a, b), cirq.CXPowGate(exponent=sym()).on(b, d),
+                  cirq.CZPowGate(exponent=sym()).on(a, d), cirq.rx(0.3 + i).on(a),
+                  cirq.ControlledGate(cirq.rx(sym()), control_values=[0]).on(d, a),
+                  cirq.ControlledGate(cirq.ry(sym()), num_controls=2).on(a, b, d), cirq.rz(0.7 * i).on(b)])
+    h = sum((float(rng.randn()) * cirq.X(q) for q in qs[1:]), float(rng.randn()) * cirq.Z(qs[0]))
+    for a, b in zip(qs, qs[1:]):
+        h = h + float(rng.randn()) * cirq.Y(a) * cirq.Z(b)
+    ag = AdjointGradient(c, h, adjoint_tile_bits=L)
+    if specialize:
+        ag.specialize()
+    x = rng.uniform(-2, 2, len(syms))
+    names = dict(zip(syms, x))
+    value, grad = ag.value_and_grad([names[s] for s in ag.symbols])
+    want = _oracle_grad(c, qs, h, ag.symbols, np.array([names[s] for s in ag.symbols]))
+    size = sum(abs(complex(t.coefficient)) for t in h)
+    print(f"  largest error {np.abs(grad - want).max() / size:.2e} of sum |c|", flush=True)
+    # complex64 states of up to 65 ops leave 3e-8 to 1.3e-7 of sum |c|, stated with four times that; the differences
+    # (h = 1e-5) are good to 1e-10
+    assert np.abs(grad - want).max() < 5e-7 * size
