@@ -310,7 +310,7 @@ def _specialize_gradient(args, ag):
 
 
 def _adjoint_roofline(ag, n_bits: int, point) -> dict:
-    """Roofline of the reverse-sweep kernel (k_adjoint_pass, the dominant one of a gradient): its
+    """Roofline of the reverse-sweep kernels (the dominant ones of a gradient): their
     algorithmic bytes per pass (psi and phi each read and written once: 4 * 8 * 2^n) over its
     average pass time, timed with HIP events on the stream the passes run on; the forward passes
     beside it (read + write once each, the first writes only)."""
@@ -322,16 +322,19 @@ def _adjoint_roofline(ag, n_bits: int, point) -> dict:
     achieved = rev_bytes / (t["reverse_ms"] / 1e3 / max(n_rev, 1)) / 1e9
     fwd_gbs = fwd_bytes / (t["forward_ms"] / 1e3 / max(n_fwd, 1)) / 1e9
     state_mib = 8 * 2**n_bits / 2**20
+    L = int(ag.prog.tile_bits_rev)
+    kernel = (f"k_aspec_* (specialised, {L}-bit tiles)" if ag.rev_spec is not None else
+              f"k_adjoint_staged<{L}> / k_adjoint_pass<{L}> (interpreted: passes of many / few ops)")
     where = ("the two states stay in the 256 MiB last-level cache" if 2 * state_mib <= 128 else
              "the two states fill the 256 MiB last-level cache and spill to HBM")
     return {
         "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-        "traffic": None, "kernel": f"k_adjoint_pass<{int(ag.prog.tile_bits_rev)}>",
+        "traffic": None, "kernel": kernel,
         "reverse_ms": t["reverse_ms"], "reverse_passes": n_rev, "forward_ms": t["forward_ms"],
         "forward_gbs": fwd_gbs,
         "note": f"{state_mib:.0f} MiB per state, {2**(n_bits - int(ag.prog.tile_bits_rev))} tiles per reverse pass: "
-        f"{where}; the passes are bound by VALU work per op (about 3 interpreted ops per parameterised gate) "
-        "and by latency at this tile count, not by HBM bandwidth",
+        f"{where}; the passes are bound by VALU work per op (two ops per parameterised gate: its generator's partial "
+        "sum and its undoing on both states) and by latency at this tile count, not by HBM bandwidth",
     }
 
 
