@@ -220,17 +220,19 @@ __device__ __forceinline__ double grad_lane1(const float2 (&x)[PER], const float
     for (int e = 0; e < PER; ++e) s = add_overlap<true>(s, f[e], x[e]);
     g = fma(-(double)d.y, s, g);
   }
-  const bool re = m01.x != 0.f || m10.x != 0.f, im = m01.y != 0.f || m10.y != 0.f;
-  if (re || im) {
-    double sr = 0.0, si = 0.0;
+  if (m01.x != 0.f || m10.x != 0.f) {
+    double s = 0.0;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const float2 p = make_float2(lane_xor<T>(x[e].x), lane_xor<T>(x[e].y));
-      if (re) sr = add_overlap<false>(sr, f[e], p);
-      if (im) si = add_overlap<true>(si, f[e], p);
-    }
-    g = fma((double)o.x, sr, g);
-    g = fma(-(double)o.y, si, g);
+    for (int e = 0; e < PER; ++e)
+      s = add_overlap<false>(s, f[e], make_float2(lane_xor<T>(x[e].x), lane_xor<T>(x[e].y)));
+    g = fma((double)o.x, s, g);
+  }
+  if (m01.y != 0.f || m10.y != 0.f) {
+    double s = 0.0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+      s = add_overlap<true>(s, f[e], make_float2(lane_xor<T>(x[e].x), lane_xor<T>(x[e].y)));
+    g = fma(-(double)o.y, s, g);
   }
   return 2.0 * g;
 }
