@@ -20,7 +20,7 @@ constexpr int kRedBlocks = 512;  // k_inner: fixed grid => deterministic reducti
 // indices: where x reaches above the chunk, half of the chunks do the work.
 // A workgroup owns a slice of the state in chunks of 2^kChunkBits amplitudes and kPauliGroup terms: it holds
 // a chunk in registers and reads each term's partner chunk i ^ x (a permutation of one chunk, so reads
-// stay coalesced; terms with equal x share it and its products), two amplitudes to a load.  The state is read about
+// stay coalesced; terms with equal x share it), two amplitudes to a load.  The state is read about
 // 1 + kPauliGroup / 2 times per kPauliGroup terms, by workgroups that run side by side (the group is the
 // fastest grid index) and find it in cache.  What bounds it is the FP64 arithmetic and, for small
 // states, the launch: 200 4-local terms on 20 qubits take 160 us
@@ -30,8 +30,8 @@ constexpr int kPauliTerms = 96;   // arguments stay below 4 KB
 constexpr int kPauliGroup = 8;    // terms of one workgroup (FP64 accumulators in registers)
 constexpr int kChunkBits = 11;    // 256 threads x 4 pairs of amplitudes
 // Slices of a state, fixed by n alone => deterministic reduction order: 512, two workgroups per CU for one group of terms;
-// 256 of two chunks and fewer below 22 qubits, where a chunk's work does not pay for reducing its sums (200 terms on 20
-// qubits: 145 us against 190).
+// at most 256 below 22 qubits, where a chunk's work does not pay for reducing its sums (200 terms on 20 qubits: 169 us
+// against 204).
 constexpr int kPauliSlices = 512;
 inline int pauli_slices(int n) {
   const int most = n >= 22 ? kPauliSlices : kPauliSlices / 2;
@@ -93,24 +93,22 @@ __global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ 
       }
     }
     float2 b[8];
-    double w[8];  // the products of the last term with another x mask, or another parity of Y
     uint64_t px = ~0ull;
-    bool podd = false;
 #pragma unroll
     for (int t = 0; t < kPauliGroup; ++t) {
       if (t >= cnt) break;
       const uint64_t x = tb.x[t0 + t], z = tb.z[t0 + t];
       // Half of the chunks for an x that leaves the chunk (sums are doubled below): of a chunk and its partner the one
       // whose bit at the top of x equals the state's top bit, or, with that in x, the one where it is clear.  The
-      // top bit numbers a slice's chunks, so every slice does its share (X on bit 12 of 29: 3.1 ms; with
-      // the lower half of each pair, the chunks of half of the slices, 3.9 ms).
+      // top bit numbers a slice's chunks, so every slice does its share (X on bit 12 of 29: 1.6 ms; taking the lower
+      // half of each pair, the chunks of half of the slices, and 256 slices 3.9 ms).
       if (!kDm && (x >> kChunkBits) != 0) {
         const int top = 63 - __builtin_clzll(x);
         if (((base >> top) ^ (top < n - 1 ? base >> (n - 1) : 0)) & 1) continue;
       }
-      const bool fresh = x != px, odd = __popcll(x & z) & 1;
-      px = x;
-      if (fresh) {
+      const bool odd = __popcll(x & z) & 1;
+      if (x != px) {
+        px = x;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const uint64_t i = base | ((uint64_t)e << 9) | (tid << 1);
@@ -130,16 +128,6 @@ __global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ 
           }
         }
       }
-      if constexpr (!kDm) {  // conj(b) a: its real part, or its imaginary part for an odd number of Y
-        if (fresh || odd != podd) {
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const double br = b[k].x * pre, bi = b[k].y * pre, xr = a[k].x * pre, xi = a[k].y * pre;
-            w[k] = odd ? fma(br, xi, -bi * xr) : fma(br, xr, bi * xi);
-          }
-        }
-        podd = odd;
-      }
       double sr = 0.0, si = 0.0;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -148,8 +136,10 @@ __global__ __launch_bounds__(256) void k_pauli_terms(const float2* __restrict__ 
         if constexpr (kDm) {
           sr = fma(sg, (double)b[k].x, sr);
           si = fma(sg, (double)b[k].y, si);
-        } else {
-          sr = fma(sg, w[k], sr);
+        } else {  // conj(b) a: its real part, or its imaginary part for an odd number of Y
+          const double br = b[k].x * pre, bi = b[k].y * pre, xr = a[k].x * pre, xi = a[k].y * pre;
+          const double w = odd ? fma(br, xi, -bi * xr) : fma(br, xr, bi * xi);
+          sr = fma(sg, w, sr);
         }
       }
       const bool neg = (((tneg >> t) & 1) ^ (__popcll(base & z) & 1)) != 0;
