@@ -12,7 +12,8 @@
 // rotation about X, Y or Z has two real numbers in its generator.  Diagonal ops on both states leave
 // conj(phi_j) psi_j as it is, so a run of them forms the products once for all its GRAD ops (specialised and decoded passes).  The reverse passes are
 // bound by VALU work and latency: a gradient of 24-node QAOA, 8 rounds (36 ZZ and 24 X rotations each), takes
-// 7.0 ms against 8.5 with dU, psi-only and phi-only ops; of the 20-qubit ansatz, 400 rotations, 2.24 against 2.74.
+// 7.1 ms against 8.5 with dU, psi-only and phi-only ops; of the 20-qubit ansatz, 400 rotations, compiled, 1.13 against
+// 1.34.
 #pragma once
 
 #include "tile.hpp"

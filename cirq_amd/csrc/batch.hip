@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void k_batch_init(float2* __restrict__ arena, 
 }
 
 // The interpreters of a batch: every workgroup decodes its program first where the width allows (96 points on
-// 8-18 qubits, values and gradients: 3.86 ms against 4.97).
+// 8-18 qubits, values and gradients: 3.98 ms against 4.97).
 template <int L>
 using BatchRun = std::conditional_t<staged_width(L), RunStaged, RunProgram>;
 template <int L>

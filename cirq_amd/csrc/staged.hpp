@@ -8,7 +8,7 @@
 // outer bits of diagonals and phases), small matrices lie in the record, and a class number selects
 // the code.  Ops without a class of their own run through the functions of tile.hpp and adjoint.hpp.
 // A one-bit gate takes 0.32 us instead of 0.74 on 10 qubits, a diagonal 0.37 instead of 0.68; the gradient of
-// a 20-qubit ansatz 1.92 ms instead of 2.24, of a 13-qubit one (4 rows) 2.04 instead of 2.50.
+// a 20-qubit ansatz 1.94 ms instead of 2.24, of a 13-qubit one (4 rows) 2.08 instead of 2.50.
 #pragma once
 
 #include "adjoint.hpp"
@@ -313,7 +313,7 @@ __device__ __forceinline__ void adjoint_staged(float2 (&va)[PER], float2 (&vb)[P
     int cls = rec_word(r, 0);
     if (cls >= kElem) {
       // a run of diagonal ops on both states, which leave the products conj(f) x as they are: formed once
-      // (DiagRun also gathers the phases, in FP64: slower here, 2.48 against 1.85 ms for the 20-qubit ansatz)
+      // (gathering the run's phases in FP64 as well was slower: 2.48 against 1.85 ms for the 20-qubit ansatz)
       double w[PER];
       double total = 0.0;
       bool have_w = false;

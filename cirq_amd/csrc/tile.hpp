@@ -579,7 +579,7 @@ __device__ __forceinline__ void reg_dense_k(float2 (&v)[PER], MPtr M, int cm, in
 // tile to LDS, waiting for the workgroup and reading it back.  An op through LDS is a chain of a
 // barrier, LDS reads, products, LDS writes and another barrier that few waves cannot hide; across
 // lanes it is 8 FMAs and at most 4 moves per amplitude.  A 14-qubit density matrix of 10 noisy layers
-// takes 12.9 ms against 13.9, a 24-node QAOA gradient 6.45 against 6.98 ms.
+// takes 12.9 ms against 13.9, a 24-node QAOA gradient 0.92 of its time through LDS.
 constexpr int kLaneBits = 6;
 
 // v of the lane whose number differs in bit T.

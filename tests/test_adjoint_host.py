@@ -167,9 +167,9 @@ def test_adjoint_rejects_measurements_and_foreign_observables():
 
 @pytest.mark.parametrize("tiles", [(3, 2), (3, 3), (4, 2)])
 def test_controlled_gradient_op_keeps_its_inverses_in_its_pass(tiles):
-    """A parameterised controlled gate whose control is outside the adjoint tile: its GRAD op needs
-    the control local, so its two one-state inverses must wait for the same pass; otherwise the
-    gradient of an earlier gate on other bits is taken while only psi has been un-computed."""
+    """A parameterised controlled gate whose control is outside the adjoint tile: its GRAD op needs the control
+    local, its undo op does not, so the two may be in different passes.  Gradients of other gates taken between
+    them must see both states with the gate or both without it."""
     b, z, c = sympy.symbols("b z c")
     q = cirq.LineQubit.range(4)
     circuit = cirq.Circuit(
