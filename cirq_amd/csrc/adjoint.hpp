@@ -7,12 +7,12 @@
 // the same at every parameter value for gates exp(i t K), and the two states stay consistent between
 // any two ops, so a gate is undone by one op instead of one per state.
 //
-// GRAD sums are sums of the products conj(phi_i) psi_j weighted by G's entries.  The products are formed
-// and summed in FP64, only those whose entry of G is not zero (a uniform test): a
-// rotation about X, Y or Z has two real numbers in its generator.  Diagonal ops on both states leave
-// conj(phi_j) psi_j as it is, so a run of them forms the products once for all its GRAD ops (specialised and decoded passes).  The reverse passes are
-// bound by VALU work and latency: a gradient of 24-node QAOA, 8 rounds (36 ZZ and 24 X rotations each), takes
-// 7.1 ms against 8.5 with dU, psi-only and phi-only ops; of the 20-qubit ansatz, 400 rotations, compiled, 1.13 against
+// GRAD sums are sums of the products conj(phi_i) psi_j weighted by G's entries.  The products are formed and
+// summed in FP64, only those whose entry of G is not zero (a uniform test): a rotation about X, Y or Z has two
+// real numbers in its generator.  Diagonal ops on both states leave conj(phi_j) psi_j as it is, so a run of them
+// forms the products once for all its GRAD ops (specialised and decoded passes).  The reverse passes are bound by
+// VALU work and latency: a gradient of 24-node QAOA, 8 rounds (36 ZZ and 24 X rotations each), takes 7.1 ms
+// against 8.5 with dU, psi-only and phi-only ops; of the 20-qubit ansatz, 400 rotations, compiled, 1.13 against
 // 1.34.
 #pragma once
 

@@ -305,8 +305,9 @@ __device__ __forceinline__ void run_staged(float2 (&v)[PER], float2* tile, float
 // adjoint.hpp's reverse pass over the records of the ops from `ops` on.
 template <int PER, int NT, int L, class Prog>
 __device__ __forceinline__ void adjoint_staged(float2 (&va)[PER], float2 (&vb)[PER], float2* tA, float2* tB,
-                                               float2* mstage, const Prog& P, const cqs_op* ops,
-                                               const int* recs, uint64_t base, bool act, double* __restrict__ partial, int64_t stride, int64_t tile) {
+                                               float2* mstage, const Prog& P, const cqs_op* ops, const int* recs,
+                                               uint64_t base, bool act, double* __restrict__ partial, int64_t stride,
+                                               int64_t tile) {
   constexpr int NR = __builtin_ctz(PER);
   for (int i = 0;; ++i) {
     const int* r = recs + i * kRecWords;
@@ -456,16 +457,18 @@ constexpr int kStagedMinL = 6, kStagedMaxL = 12;
 constexpr int kStagedAdjMaxL = 11;  // two states of 16 elements per thread spill 400 registers here
 constexpr bool staged_adjoint_width(int L) { return L >= kStagedMinL && L <= kStagedAdjMaxL; }
 constexpr bool staged_width(int L) { return L >= kStagedMinL && L <= kStagedMaxL; }
+
 // Passes that are decoded first: those of many ops.  Decoding costs a start (0.3-1 us on few tiles, a tenth of a
-// pass of 2-4 ops) and 0.1-0.2 us more for each op without a class of its own, and saves 0.2-0.4 us for each op with one.  The
-// host does not see the kinds (ops lie on the device), but programs of one-bit gates have long passes, and those whose gates
-// fuse into two-bit matrices and MFMA blocks short ones: grid circuits and noisy density matrices 1-14 ops.  Scalar /
-// decoded in us: 16 one-bit and diagonal ops 14.0 / 10.2 on 10 qubits, 23.0 / 18.1 on 20, 31.3 / 31.0 on 22; 8 blocks and
-// phases 10.9 / 11.4, 19.7 / 20.4, 30.2 / 33.2; 16 of them 19.1 / 19.0, 34.2 / 34.5, 52.5 / 56.3.  On more tiles the waves hide
-// more of the scalar decoding: 16 gates 56 / 54 on 23 qubits, 368 / 357 on 26, 32 gates 100 / 91 and 689 / 627.
-// The same in reverse passes: 8 gates and gradients 12.6 / 9.2 on 10 qubits, 18.0 / 15.3 on 20, 130 / 132 on 24, 16 of
-// them 22.1 / 13.8, 29.2 / 22.2, 226 / 201; 4 blocks 11.7 / 13.0, 17.4 / 19.5, 145 / 187, 16 blocks, gradients and phases
-// 29.5 / 25.8, 38.8 / 38.5, 335 / 392, 32 of them 54.4 / 44.9, 68.5 / 66.2, 617 / 702.
+// pass of 2-4 ops) and 0.1-0.2 us more for each op without a class of its own, and saves 0.2-0.4 us for each op
+// with one.  The host does not see the kinds (ops lie on the device), but programs of one-bit gates have long
+// passes, and those whose gates fuse into two-bit matrices and MFMA blocks short ones: grid circuits and noisy
+// density matrices 1-14 ops.  Scalar / decoded in us: 16 one-bit and diagonal ops 14.0 / 10.2 on 10 qubits, 23.0 /
+// 18.1 on 20, 31.3 / 31.0 on 22; 8 blocks and phases 10.9 / 11.4, 19.7 / 20.4, 30.2 / 33.2; 16 of them 19.1 /
+// 19.0, 34.2 / 34.5, 52.5 / 56.3.  On more tiles the waves hide more of the scalar decoding: 16 gates 56 / 54 on
+// 23 qubits, 368 / 357 on 26, 32 gates 100 / 91 and 689 / 627. The same in reverse passes: 8 gates and gradients
+// 12.6 / 9.2 on 10 qubits, 18.0 / 15.3 on 20, 130 / 132 on 24, 16 of them 22.1 / 13.8, 29.2 / 22.2, 226 / 201; 4
+// blocks 11.7 / 13.0, 17.4 / 19.5, 145 / 187, 16 blocks, gradients and phases 29.5 / 25.8, 38.8 / 38.5, 335 / 392,
+// 32 of them 54.4 / 44.9, 68.5 / 66.2, 617 / 702.
 constexpr int kStagedOuterBits = 10, kStagedOps = 16, kStagedManyOps = 32;
 inline bool staged_ops(const TileProg& P) {
   return P.op_count >= (P.nouter <= kStagedOuterBits ? kStagedOps : kStagedManyOps);
